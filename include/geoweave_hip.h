@@ -525,6 +525,32 @@ int gw_sparse_attn_fwd_dense_noalloc(int dtype,
                                      void* stream);
 
 /* ------------------------------------------------------------------------------------
+ * Sparse-index attention forward over per-block key unions (inference: o and lse, no
+ * attn_sum): the same results as gw_sparse_attn_fwd up to fp32 summation order and the fp16
+ * rounding of P. Sixteen queries of a head form products with the keys that at least one of
+ * them selected, 1 - (1 - K / S)^16 of all keys for spread selections; it pays off over
+ * gw_sparse_attn_fwd_dense where a query selects less than about one key in eight.
+ * Needs D = 64 and softmax_scale * log2(e) in [2^-60, 2^60]; otherwise GW_ERR_UNSUPPORTED.
+ * Queries that list a position twice, and batch elements with a non-finite K or V value, are
+ * computed by the gather kernel inside this call. lse may be null.
+ * Workspace: gw_sparse_attn_fwd_union_workspace_size(B, T, S, H, D, K) bytes, 16-byte aligned
+ * (selection records, B * round_up(T, 256) / 16 * ceil(S / 256) * 1024 bytes; the tiled K and
+ * fp16 V, B * H * ceil(S / 256) * 65536 bytes; flags and |V| column maxima).
+ * ------------------------------------------------------------------------------------ */
+size_t gw_sparse_attn_fwd_union_workspace_size(int64_t B, int64_t T, int64_t S, int64_t H, int64_t D,
+                                               int64_t K);
+int gw_sparse_attn_fwd_union(int dtype,
+                             const void* q, const int64_t* q_strides,
+                             const void* k, const int64_t* k_strides,
+                             const void* v, const int64_t* v_strides,
+                             const int32_t* kv_pos, int64_t pos_stride_b, int64_t pos_stride_t,
+                             void* o, const int64_t* o_strides, float* lse,
+                             int64_t B, int64_t T, int64_t S, int64_t H, int64_t D, int64_t K,
+                             float softmax_scale,
+                             void* workspace, size_t workspace_bytes,
+                             void* stream);
+
+/* ------------------------------------------------------------------------------------
  * Sparse-index attention backward as masked dense passes: the same gradients as
  * gw_sparse_attn_bwd without an attn_sum gradient (dq, dk, dv up to fp32 summation order and
  * the rounding of P and dS to the input type for their matrix products), computed on the

@@ -1,0 +1,143 @@
+"""GPU parity of the union attention forward (gw_sparse_attn_fwd_union) against the oracle.
+
+Sixteen queries of a head share one list of keys per 256-key tile (at most 8 steps of 32
+keys, in two groups of 4), so the sizes here sit at the edges of blocks, tiles, steps and
+groups, and the positions range from a few keys per tile to every key of it.
+
+Tolerance: P enters its product as fp16 (relative error 2^-11 per weight), V as fp16 (2^-11;
+exact for fp16 inputs up to the scaling), o is rounded to the input type (2^-9 in bf16, 2^-12
+in fp16); the 2-norm of independent roundings stays below the sum of the three bounds. lse: an
+fp32 sum of fp32 weights (1e-5) over fp32 scores, which both sides sum over 64 products (a
+random walk of 64 roundings is 8 ulp a side: 16 ulp = 2^-20 of |lse|, the scores' size).
+"""
+import contextlib
+
+import pytest
+import torch
+
+from geoweave_amd.custom_flash_attn import sparse_index_flash_attn as sifa
+from oracle import attention as oatt
+
+pytestmark = pytest.mark.gpu
+
+REL = {torch.bfloat16: 2.0 ** -9 + 2.0 ** -10, torch.float16: 2.0 ** -12 + 2.0 ** -10}
+
+
+@contextlib.contextmanager
+def _path(name):
+    old = sifa.FORWARD_PATH
+    sifa.FORWARD_PATH = name
+    try:
+        yield
+    finally:
+        sifa.FORWARD_PATH = old
+
+
+def _inputs(B, T, S, H, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(B, n, H, 64, generator=g).to(dtype) for n in (T, S, S)]
+
+
+def _positions(B, T, S, K, seed, lo=0, hi=None):
+    """Distinct positions in [lo, hi) per row."""
+    g = torch.Generator().manual_seed(seed)
+    hi = S if hi is None else hi
+    return (lo + torch.rand(B, T, hi - lo, generator=g).topk(K, dim=-1).indices).to(torch.int32)
+
+
+def _run(q, k, v, pos, scale=0.125, layout="bthd", path="union"):
+    qd, kd, vd, pd = (x.cuda() for x in (q, k, v, pos))
+    if layout == "bhtd":
+        qd, kd, vd = (x.transpose(1, 2).contiguous() for x in (qd, kd, vd))
+    with _path(path):
+        o, attn, lse, _ = sifa._flash_attn_forward(qd, kd, vd, pd, softmax_scale=scale, return_attn=False, q_layout=layout)
+    torch.cuda.synchronize()
+    assert attn is None
+    return (o.transpose(1, 2) if layout == "bhtd" else o).float().cpu(), lse.cpu()
+
+
+def _check(q, k, v, pos, o, lse, scale=0.125):
+    ro, _, rl = oatt.sparse_attention(q.float(), k.float(), v.float(), pos, scale)
+    assert torch.equal(torch.isinf(lse), torch.isinf(rl))
+    ok = torch.isfinite(rl)
+    assert ((lse[ok] - rl[ok]).abs() <= 1e-5 + 2.0 ** -20 * rl[ok].abs()).all()
+    assert torch.isfinite(o).all()
+    assert (o - ro).norm() <= REL[q.dtype] * ro.norm()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,S,K", [(1, 1, 1), (15, 255, 7), (16, 256, 256), (17, 257, 40), (255, 513, 16), (257, 700, 300),
+                                   (529, 1025, 64), (40, 5000, 600)])
+def test_edges(gpu_device, dtype, T, S, K):
+    print(f"[union] T={T} S={S} K={K} {dtype}", flush=True)
+    q, k, v = _inputs(2, T, S, 3, dtype, T * 31 + S)
+    pos = _positions(2, T, S, K, S)
+    _check(q, k, v, pos, *_run(q, k, v, pos))
+
+
+@pytest.mark.parametrize("lo,width,K", [(0, 256, 100), (256, 256, 9), (512, 200, 128), (100, 300, 64), (768, 32, 5)])
+def test_clustered_positions(gpu_device, lo, width, K):
+    # Whole tiles listed by the block (both groups of steps), one step, and tiles with none.
+    print(f"[union] clustered lo={lo} width={width} K={K}", flush=True)
+    q, k, v = _inputs(1, 130, 1100, 2, torch.bfloat16, lo + K)
+    pos = _positions(1, 130, 1100, K, K, lo, lo + width)
+    _check(q, k, v, pos, *_run(q, k, v, pos))
+
+
+def test_masked_empty_and_growing_scores(gpu_device):
+    # -1 and out-of-range positions, rows without any, and scores that rise along the keys (the
+    # reference maximum moves many times).
+    print("[union] masked", flush=True)
+    q, k, v = _inputs(1, 100, 2000, 2, torch.float16, 5)
+    q = q.abs() * 4
+    k = (k.abs() * torch.linspace(0.1, 4, 2000).view(1, -1, 1, 1)).to(torch.float16)
+    pos = _positions(1, 100, 2000, 90, 6)
+    pos[:, ::3, 40:] = -1
+    pos[:, 7] = -1
+    pos[:, 9, 5:] = 5000
+    o, lse = _run(q, k, v, pos)
+    _check(q, k, v, pos, o, lse)
+    assert (o[:, 7] == 0).all()
+
+
+def test_repeated_positions_and_nonfinite_rows(gpu_device):
+    # Both are computed by the gather kernel inside the call.
+    print("[union] repeated, non-finite", flush=True)
+    q, k, v = _inputs(2, 70, 900, 2, torch.bfloat16, 11)
+    pos = _positions(2, 70, 900, 50, 12, 0, 899)
+    pos[0, 33, 1] = pos[0, 33, 0]
+    _check(q, k, v, pos, *_run(q, k, v, pos))
+    k2, v2 = k.clone(), v.clone()
+    k2[1, 899], v2[1, 899] = float("nan"), float("inf")  # a row that no query selected
+    _check(q, k, v, pos, *_run(q, k2, v2, pos))
+
+
+@pytest.mark.parametrize("layout", ["bthd", "bhtd"])
+def test_layouts_strides_and_column_scales(gpu_device, layout):
+    print(f"[union] {layout}", flush=True)
+    q, k, v = _inputs(1, 90, 1300, 4, torch.bfloat16, 21)
+    v = (v.float() * torch.logspace(-6, 6, 64)).to(torch.bfloat16)
+    pos = _positions(1, 90, 1300, 70, 22)
+    o, lse = _run(q, k, v, pos, layout=layout)
+    ro, _, _ = oatt.sparse_attention(q.float(), k.float(), v.float(), pos, 0.125)
+    col = lambda x: x.reshape(-1, 64).norm(dim=0)  # noqa: E731
+    assert (col(o - ro) <= REL[torch.bfloat16] * col(ro)).all()
+    if layout == "bthd":  # strided views (v read in place from a wider row), positions with a row stride
+        wide = torch.zeros(1, 1300, 4 * 64 * 2, dtype=torch.bfloat16)
+        wide[..., 256:] = v.reshape(1, 1300, 256)
+        vv = wide.cuda()[..., 256:].view(1, 1300, 4, 64)
+        pp = torch.cat([pos, pos], -1).cuda()[..., :70]
+        with _path("union"):
+            o2, _, lse2, _ = sifa._flash_attn_forward(q.cuda(), k.cuda(), vv, pp, softmax_scale=0.125, return_attn=False)
+        assert torch.equal(o2.float().cpu(), o) and torch.equal(lse2.cpu(), lse)
+
+
+def test_routes(gpu_device):
+    # The rule's own choice agrees with the gather kernel on both sides of its line.
+    for S, K in ((16 * 64, 64), (18 * 64, 64), (97 * 64, 64)):
+        print(f"[union] route S={S} K={K}", flush=True)
+        q, k, v = _inputs(1, 64, S, 2, torch.bfloat16, S)
+        pos = _positions(1, 64, S, K, S)
+        o, lse = _run(q, k, v, pos, path="auto")
+        og, lg = _run(q, k, v, pos, path="gather")
+        assert (o - og).norm() <= 2 * REL[torch.bfloat16] * og.norm() and (lse - lg).abs().max() < 1e-4
