@@ -795,6 +795,11 @@ struct SelectParams {
   int* wide_list;
   int64_t rows;
   int force_wide;  // test hook: every complete row takes the LDS selection
+  // ROWS kernels: the scores of every key, [rows][S], and the threshold of the marks (-inf).
+  const float* full;
+  int S;
+  int bn;  // keys per filter stage (64 or 32): the order of the entries
+  float tau0;
 };
 
 // Number of set bits of a wave mask below this lane.
@@ -842,15 +847,41 @@ __device__ __forceinline__ bool row_lists(const SelectParams& p, int64_t row, Ro
   return bad;
 }
 
-template <typename E, int KS>
+// ROWS: the candidates are all keys, their scores read from a score row instead of lists (short
+// key sets, see Plan::rows_all). The entries keep the lists' order: entry 64 m + l of a row is
+// the key that the filter's lane half l / 32 holds as element l % 16 of tile l % 32 / 16 of
+// stage m (stages of 64 keys; of 32: half l % 32 / 16, stage 2 m + l / 32), and keys that the filter would not mark (score - inf, or NaN) stay out.
+template <typename E, int KS, bool ROWS>
 __global__ __launch_bounds__(256) void indexer_select_kernel(const SelectParams p) {
   __shared__ uint32_t cbuf[4][kCompactKeys];
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (row >= p.rows) return;
+  uint32_t kv[KS];
+  int32_t ky[KS];
   RowLists rl;
-  const bool bad = row_lists(p, row, rl);
-  const int total = rl.off[kMaxLists];
+  bool bad = false;
+  int total = 0;
+  if constexpr (ROWS) {
+    const float* sc = p.full + row * p.S;
+    const int k0 = (p.bn == 64 ? 2 * (lane & 16) + 4 * (lane >> 5) : (lane & 32) + ((lane & 16) >> 2)) +
+                   8 * ((lane & 15) >> 2) + (lane & 3);
+#pragma unroll
+    for (int m = 0; m < KS; ++m) {
+      ky[m] = 64 * m + k0;
+      kv[m] = ky[m] < p.S ? __float_as_uint(sc[ky[m]]) : 0u;
+    }
+#pragma unroll
+    for (int m = 0; m < KS; ++m) {
+      const float v = __uint_as_float(kv[m]);
+      const bool live = ky[m] < p.S && (int32_t)__float_as_uint(p.tau0 - v) < 0;
+      total += __popcll(__ballot(live));
+      kv[m] = live ? f2key(v) : 0u;
+    }
+  } else {
+    bad = row_lists(p, row, rl);
+    total = rl.off[kMaxLists];
+  }
   if (bad || total < p.Kk) {
     // The candidates may miss part of the top-k: exact brute force.
     if (lane == 0) {
@@ -859,12 +890,12 @@ __global__ __launch_bounds__(256) void indexer_select_kernel(const SelectParams 
     }
     return;
   }
-  if (p.force_wide || total > 64 * KS) {
+  if (!ROWS && (p.force_wide || total > 64 * KS)) {
     // Complete candidates, more than the registers hold: the LDS selection.
     if (lane == 0) p.wide_list[atomicAdd(p.wide_count, 1)] = (int)row;
     return;
   }
-  const int nch = (total + 63) / 64;  // register slots in use, uniform
+  const int nch = ((ROWS ? p.S : total) + 63) / 64;  // register slots in use, uniform
 
   // Slots past the end hold key 0, below the key of every finite score; chunks of 8 slots
   // past the last one in use are skipped with a uniform branch.
@@ -872,9 +903,8 @@ __global__ __launch_bounds__(256) void indexer_select_kernel(const SelectParams 
   // output, so the list position of an entry is computed once.
   // All loads are issued before any is used (the score bits land in kv and become keys in a
   // second pass), so the chunks of 8 slots do not wait for each other.
-  uint32_t kv[KS];
-  int32_t ky[KS];
   uint32_t lmin = 0xFFFFFFFFu, lmax = 0u;
+  if constexpr (!ROWS) {
 #pragma unroll
   for (int m0 = 0; m0 < KS; m0 += 8) {
 #pragma unroll
@@ -901,6 +931,7 @@ __global__ __launch_bounds__(256) void indexer_select_kernel(const SelectParams 
       for (int m = m0; m < m0 + 8; ++m)
         if (m * 64 + lane < total) kv[m] = f2key(__uint_as_float(kv[m]));
     }
+  }
   }
   // Key range of the live slots: empty slots hold 0, which kv - 1 wraps to the maximum (the
   // + 1 comes after the wave minimum, so a lane without live slots does not wrap back to 0).
@@ -1301,6 +1332,11 @@ struct Plan {
   int Kk = 0;
   bool sample = false;
   bool full_all = false;  // every row through the full scoring and the row select
+  // Without a sampled threshold every key is a candidate: the scores of all keys go to rows (the
+  // key range split over the chip) and the register select reads those. The filter would
+  // write them as candidate lists, one lane's marks at a time, from one key split: 438 us of
+  // the 480 us a call with 2,748 queries and keys took; 27 + 33 us as rows.
+  bool rows_all = false;
   int full_rows = 0;      // rows per batch element scored per round on the full path
   int Ms = 0, rank = 0;
   int nsplit = 1, cap = 0;
@@ -1460,6 +1496,8 @@ template <typename E, int HI, int BIAS>
 int run_typed(const ScoreParams& base, Plan pl, int64_t B, int32_t* out_idx, void* out_scores,
               uint8_t* ws, hipStream_t st) {
   if (pl.full_all) return run_full_rows<E, HI, BIAS>(base, pl, B, out_idx, out_scores, ws, st);
+  // The test hooks (forced thresholds, forced LDS selection) act on the candidate lists.
+  pl.rows_all = !pl.sample && base.tau_mode == kTauArray && base.force_wide == 0;
   int* counters = reinterpret_cast<int*>(ws + pl.off_fb);  // [0] wide select, [1 + b] fallback of b
   hipLaunchKernelGGL(set_ints_kernel, dim3(1), dim3(256), 0, st, counters, (int)B + 1, 0);
   GW_HIP_LAUNCH_CHECK("set_ints_kernel");
@@ -1495,6 +1533,21 @@ int run_typed(const ScoreParams& base, Plan pl, int64_t B, int32_t* out_idx, voi
       hipLaunchKernelGGL((indexer_tau_kernel<32>), tgrid, dim3(256), 0, st, sp.samp, pl.Ms, pl.rank, 8, tau, rows);
     GW_HIP_LAUNCH_CHECK("indexer_tau_kernel");
   }
+  if (pl.rows_all) {
+    // Scores of every key, [rows][S] in the candidate lists' space (S <= kSubTotal / 2). The key
+    // range splits into as many parts as fill the chip twice, of two stages at least.
+    ScoreParams sp = base;
+    sp.samp = reinterpret_cast<float*>(ws + pl.off_cand);
+    sp.Ms = base.S;
+    sp.tau = nullptr;
+    sp.nstages = (base.S + BN - 1) / BN;
+    const int slots = filter_slots((const void*)indexer_score_kernel<E, HI, true, BIAS>, THREADS);
+    const int64_t want = (2 * (int64_t)slots + tiles * B - 1) / (tiles * B);
+    sp.nsplit = (int)std::max<int64_t>(1, std::min<int64_t>(want, std::max(1, sp.nstages / 2)));
+    hipLaunchKernelGGL((indexer_score_kernel<E, HI, true, BIAS>),
+                       dim3((unsigned)tiles, (unsigned)sp.nsplit, (unsigned)B), dim3(THREADS), 0, st, sp);
+    GW_HIP_LAUNCH_CHECK("indexer_score_kernel<all keys>");
+  }
   ScoreParams fp = base;
   fp.tau = pl.sample ? tau : nullptr;
   fp.cand = reinterpret_cast<int2*>(ws + pl.off_cand);
@@ -1502,9 +1555,11 @@ int run_typed(const ScoreParams& base, Plan pl, int64_t B, int32_t* out_idx, voi
   fp.nsplit = pl.nsplit;
   fp.cap = pl.cap;
   fp.nstages = (base.S + BN - 1) / BN;
-  hipLaunchKernelGGL((indexer_score_kernel<E, HI, false, BIAS>),
-                     dim3((unsigned)tiles, (unsigned)pl.nsplit, (unsigned)B), dim3(THREADS), 0, st, fp);
-  GW_HIP_LAUNCH_CHECK("indexer_score_kernel<filter>");
+  if (!pl.rows_all) {
+    hipLaunchKernelGGL((indexer_score_kernel<E, HI, false, BIAS>),
+                       dim3((unsigned)tiles, (unsigned)pl.nsplit, (unsigned)B), dim3(THREADS), 0, st, fp);
+    GW_HIP_LAUNCH_CHECK("indexer_score_kernel<filter>");
+  }
   SelectParams fs{};
   fs.cand = fp.cand;
   fs.counts = fp.counts;
@@ -1521,6 +1576,10 @@ int run_typed(const ScoreParams& base, Plan pl, int64_t B, int32_t* out_idx, voi
   fs.wide_list = reinterpret_cast<int*>(ws + pl.off_widelist);
   fs.rows = rows;
   fs.force_wide = base.force_wide;
+  fs.full = reinterpret_cast<const float*>(ws + pl.off_cand);
+  fs.S = base.S;
+  fs.bn = BN;
+  fs.tau0 = -INFINITY;
   const dim3 sgrid2((unsigned)((rows + 3) / 4));
   // Register slots: the fewest that hold 1.25 x the expected candidates per query plus five
   // Poisson deviations (the largest tier when none does: rows beyond it take the LDS
@@ -1529,15 +1588,27 @@ int run_typed(const ScoreParams& base, Plan pl, int64_t B, int32_t* out_idx, voi
   // took 2.87 instead of 2.12 ms.
   const double expect = pl.sample ? (double)pl.rank * (double)base.S / (double)pl.Ms : (double)base.S;
   const double need = 1.25 * expect + 5.0 * std::sqrt(expect);
-  if (need <= 64.0 * kSelRegsTiers[0])
-    hipLaunchKernelGGL((indexer_select_kernel<E, kSelRegsTiers[0]>), sgrid2, dim3(256), 0, st, fs);
-  else if (need <= 64.0 * kSelRegsTiers[1])
-    hipLaunchKernelGGL((indexer_select_kernel<E, kSelRegsTiers[1]>), sgrid2, dim3(256), 0, st, fs);
-  else
-    hipLaunchKernelGGL((indexer_select_kernel<E, kSelRegsTiers[2]>), sgrid2, dim3(256), 0, st, fs);
-  GW_HIP_LAUNCH_CHECK("indexer_select_kernel");
-  hipLaunchKernelGGL((indexer_select_wide_kernel<E>), dim3(kFallbackBlocks), dim3(256), 0, st, fs);
-  GW_HIP_LAUNCH_CHECK("indexer_select_wide_kernel");
+  if (pl.rows_all) {
+    // One slot per key: 1,536, 3,072 or 4,096 of them.
+    static_assert(kSubTotal / 2 <= 64 * 64, "a row's keys fit the largest tier");
+    if (base.S <= 64 * 24)
+      hipLaunchKernelGGL((indexer_select_kernel<E, 24, true>), sgrid2, dim3(256), 0, st, fs);
+    else if (base.S <= 64 * 48)
+      hipLaunchKernelGGL((indexer_select_kernel<E, 48, true>), sgrid2, dim3(256), 0, st, fs);
+    else
+      hipLaunchKernelGGL((indexer_select_kernel<E, 64, true>), sgrid2, dim3(256), 0, st, fs);
+    GW_HIP_LAUNCH_CHECK("indexer_select_kernel<rows>");
+  } else {
+    if (need <= 64.0 * kSelRegsTiers[0])
+      hipLaunchKernelGGL((indexer_select_kernel<E, kSelRegsTiers[0], false>), sgrid2, dim3(256), 0, st, fs);
+    else if (need <= 64.0 * kSelRegsTiers[1])
+      hipLaunchKernelGGL((indexer_select_kernel<E, kSelRegsTiers[1], false>), sgrid2, dim3(256), 0, st, fs);
+    else
+      hipLaunchKernelGGL((indexer_select_kernel<E, kSelRegsTiers[2], false>), sgrid2, dim3(256), 0, st, fs);
+    GW_HIP_LAUNCH_CHECK("indexer_select_kernel");
+    hipLaunchKernelGGL((indexer_select_wide_kernel<E>), dim3(kFallbackBlocks), dim3(256), 0, st, fs);
+    GW_HIP_LAUNCH_CHECK("indexer_select_wide_kernel");
+  }
   // Rows queued for the exact fallback (sampled threshold too high or a list overflowed):
   // scores over all keys on the matrix cores, rows gathered from the queue, key range split
   // finely so that a few hundred rows still fill the chip (workgroups of batch elements with
