@@ -6,8 +6,8 @@
 // keys selected per query that is 1 - (1 - r)^16 of them (31 % at 1,024 of 43,968 keys, 17 %
 // at 1,024 of 87,936), so matrix work, exponentials and operand reads all shrink by that
 // factor, while each K and V row is still read from memory once per workgroup (up to 512
-// queries) and shared through LDS. With 16 heads the whole call takes 4.6 ms against the
-// dense pass's 7.45 ms at 43,968 keys (K = 1,024) and 12.5 ms against 28.4 ms at 87,936.
+// queries) and shared through LDS. With 16 heads the whole call takes 4.34 ms against the
+// dense pass's 7.45 ms at 43,968 keys (K = 1,024) and 11.8 ms against 28.4 ms at 87,936.
 //
 // Pieces (all on the caller's stream):
 //   union_lists_kernel  - the (block, tile) records of gw_union.h from the positions; a position
@@ -20,6 +20,8 @@
 //                         the LDS image of a tile, so that staging a tile is one contiguous copy.
 //   union_attn_kernel   - the attention.
 #include <math.h>
+
+#include <type_traits>
 
 #include "gw_attn.h"
 #include "gw_common.h"
@@ -225,7 +227,9 @@ __global__ __launch_bounds__(256) void union_tiles_kernel(const uint16_t* __rest
 // of 32 queries is 1.7 times as large at these sizes, so the exponentials grow by that while
 // only the LDS reads shrink. Tiles of 256 keys: the largest that fit twice. Lists through
 // buffer loads two tiles ahead (a flat load also counts as an LDS access, and every operand
-// read waits for it).
+// read waits for it). A tile's last step takes 16 slots when the rest are empty (4.6 -> 4.34 ms).
+// Measured and not kept: the selection as a 4-bit-float matrix product instead of eight bit
+// selects a step (4.52 ms: the product sits at the head of the step's dependent chain).
 // ---------------------------------------------------------------------------------------
 constexpr float kUSumCap = 32768.f;
 
@@ -342,43 +346,47 @@ __global__ __launch_bounds__(1024) void union_attn_kernel(const UnionParams p) {
   const uint32_t vx = lds0 + (((uint32_t)i16 >> 1 & 1u) << 4) + (((uint32_t)i16 & 1u) << 3) + 2 * kUPlane;
   const uint32_t ko = (uint32_t)i16 * 4u, vo = (uint32_t)(4 * g + (i16 >> 2)) * 4u;
 
-  // One step of block a: w holds the step's bits at bits 7 (slots 0-15) and 6 (slots 16-31) of
-  // its bytes.
-  auto step = [&](int a, uint32_t w, uint32_t kr, uint32_t vr, uint32_t kl, uint32_t vl) __attribute__((always_inline)) {
-    uint4 ka[2][2];
-    uint2 va[4][2];
+  // One step of block a, its 32 slots or (half a step, F = 1) its first 16: w holds the step's
+  // bits at bits 7 (slots 0-15) and 6 (slots 16-31) of its bytes.
+  auto step = [&](auto fc, int a, uint32_t w, uint32_t kr, uint32_t vr, uint32_t kl, uint32_t vl) __attribute__((always_inline)) {
+    constexpr int F = decltype(fc)::value;
+    uint4 ka[F][2];
+    uint2 va[4][F];
     const uint32_t wb[2] = {w, w << 1};
     const uint32_t kro[2] = {kr & 0xFFFFu, kr >> 16}, vro[2] = {vr & 0xFFFFu, vr >> 16};
 #pragma unroll
-    for (int f = 0; f < 2; ++f) {
+    for (int f = 0; f < F; ++f) {
       const uint32_t at = kro[f] ^ kl;
       ka[f][0] = lds_read16(at);
       ka[f][1] = lds_read16(at + kUPlane);
     }
 #pragma unroll
-    for (int f = 0; f < 2; ++f) {
+    for (int f = 0; f < F; ++f) {
       const uint32_t at = vro[f] ^ vl, at2 = at ^ 32u;
       va[0][f] = lds_read_tr(at);
       va[1][f] = lds_read_tr(at2);
       va[2][f] = lds_read_tr(at + kUPlane);
       va[3][f] = lds_read_tr(at2 + kUPlane);
     }
-    f32x4 s[2];
+    f32x4 s[F];
 #pragma unroll
-    for (int f = 0; f < 2; ++f)
+    for (int f = 0; f < F; ++f)
 #pragma unroll
       for (int j = 0; j < 4; ++j) s[f][j] = select_bias16(wb[f], j);
 #pragma unroll
-    for (int f = 0; f < 2; ++f) s[f] = mma16(E{}, ka[f][0], qb[a][0], s[f]);
+    for (int f = 0; f < F; ++f) s[f] = mma16(E{}, ka[f][0], qb[a][0], s[f]);
 #pragma unroll
-    for (int f = 0; f < 2; ++f) s[f] = mma16(E{}, ka[f][1], qb[a][1], s[f]);
-    float pv[2][4];
+    for (int f = 0; f < F; ++f) s[f] = mma16(E{}, ka[f][1], qb[a][1], s[f]);
+    float pv[F][4];
     auto weights = [&](float nm) __attribute__((always_inline)) {
+      float t[F];
 #pragma unroll
-      for (int f = 0; f < 2; ++f)
+      for (int f = 0; f < F; ++f) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) pv[f][j] = fexp2(fmaf(s[f][j], sl2, nm));
-      return ((pv[0][0] + pv[0][1]) + (pv[0][2] + pv[0][3])) + ((pv[1][0] + pv[1][1]) + (pv[1][2] + pv[1][3]));
+        t[f] = (pv[f][0] + pv[f][1]) + (pv[f][2] + pv[f][3]);
+      }
+      return F == 2 ? t[0] + t[F - 1] : t[0];
     };
     float ls = weights(-m[a]);
     if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(ls <= kUSumCap)) != 0ull, 0)) {
@@ -386,7 +394,7 @@ __global__ __launch_bounds__(1024) void union_attn_kernel(const UnionParams p) {
       // if that is higher; O and the row sum are rescaled and the weights formed again.
       float mx = -INFINITY;
 #pragma unroll
-      for (int f = 0; f < 2; ++f)
+      for (int f = 0; f < F; ++f)
 #pragma unroll
         for (int j = 0; j < 4; ++j) mx = fmaxf(mx, s[f][j]);
       mx = pair_max(row_max(mx));
@@ -401,11 +409,14 @@ __global__ __launch_bounds__(1024) void union_attn_kernel(const UnionParams p) {
       ls = weights(-mn);
     }
     l[a] += ls;
-    const uint4 pb = make_uint4(pack_f16(pv[0][0], pv[0][1]), pack_f16(pv[0][2], pv[0][3]), pack_f16(pv[1][0], pv[1][1]),
-                                pack_f16(pv[1][2], pv[1][3]));
+    uint4 pb = make_uint4(pack_f16(pv[0][0], pv[0][1]), pack_f16(pv[0][2], pv[0][3]), 0u, 0u);
+    if constexpr (F == 2) {
+      pb.z = pack_f16(pv[1][0], pv[1][1]);
+      pb.w = pack_f16(pv[1][2], pv[1][3]);
+    }
 #pragma unroll
     for (int d = 0; d < 4; ++d)
-      acc[a][d] = mma16(FP16{}, make_uint4(va[d][0].x, va[d][0].y, va[d][1].x, va[d][1].y), pb, acc[a][d]);
+      acc[a][d] = mma16(FP16{}, make_uint4(va[d][0].x, va[d][0].y, va[d][F - 1].x, va[d][F - 1].y), pb, acc[a][d]);
   };
 
   // Tile n is in LDS buffer n % 2; while it is computed, tile n + 1's rows go to the other
@@ -429,11 +440,11 @@ __global__ __launch_bounds__(1024) void union_attn_kernel(const UnionParams p) {
   };
   // Row offsets of a tile's list to LDS (odd or even half of the wave's rows), its step counts,
   // and the rows of its first steps.
-  auto put_rows = [&](const List& x, uint32_t half, int (&ns)[NB], uint32_t (&kr)[NB], uint32_t (&vr)[NB]) __attribute__((always_inline)) {
+  auto put_rows = [&](const List& x, uint32_t half, int (&un)[NB], uint32_t (&kr)[NB], uint32_t (&vr)[NB]) __attribute__((always_inline)) {
 #pragma unroll
     for (int a = 0; a < NB; ++a) {
       const uint32_t c = (uint32_t)__builtin_amdgcn_readfirstlane(x.pr[a]);
-      ns[a] = blk[a] < p.nblk ? (int)(((c & 15u) | ((c >> 12) & 16u)) + 1u) >> 1 : 0;
+      un[a] = blk[a] < p.nblk ? (int)((c & 15u) | ((c >> 12) & 16u)) : 0;
       const uint32_t at = pl + half + 256u * a;
       lds_write4(at + (uint32_t)lane * 4u, x.pr[a] & 0xFFF0FFF0u);
       kr[a] = lds_read4(at + ko);
@@ -441,14 +452,14 @@ __global__ __launch_bounds__(1024) void union_attn_kernel(const UnionParams p) {
     }
   };
   List cur, nxt;
-  int ns[NB];
+  int un[NB];  // units of 16 slots
   uint32_t kr0[NB], vr0[NB];
   load_list(0, cur);
   load_list(1, nxt);
   stage(0, lds0);
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
-  put_rows(cur, 0u, ns, kr0, vr0);
+  put_rows(cur, 0u, un, kr0, vr0);
   __syncthreads();
 #pragma unroll 1
   for (int n = 0; n < ntiles; ++n) {
@@ -458,28 +469,28 @@ __global__ __launch_bounds__(1024) void union_attn_kernel(const UnionParams p) {
 #pragma unroll
     for (int a = 0; a < NB; ++a) {
       w1[a] = pr1[a] = 0u;
-      if (ns[a] > 4) {
+      if (un[a] > 8) {
         const char* r = rec[a] + (int64_t)n * kURec;
         w1[a] = buffer_load4(r, (uint32_t)lane * 4u + 256u);
         pr1[a] = buffer_load4(r, (uint32_t)lane * 4u + 768u);
       }
     }
     List aft;
-    int nsn[NB];
+    int unn[NB];
     uint32_t krn[NB], vrn[NB];
 #pragma unroll
     for (int a = 0; a < NB; ++a) {
       uint32_t w = cur.w[a], kr = kr0[a], vr = vr0[a];
       const uint32_t pa = pl + half + 256u * a;
       uint32_t pk = pa + ko + 64u, pv = pa + vo + 64u;
-      // One step and the next one's rows (past the last step: not used).
+      // A whole step and the next one's rows (past the last step: not used).
       auto next_step = [&](int s) __attribute__((always_inline)) {
         uint32_t kr2 = lds_read4(pk), vr2 = lds_read4(pv);
-        step(a, w, kr, vr, kx + bo, vx + bo);
+        step(std::integral_constant<int, 2>{}, a, w, kr, vr, kx + bo, vx + bo);
         pk += 64u;
         pv += 64u;
         w <<= 2;
-        if (s == 3 && ns[a] > 4) {
+        if (s == 3 && un[a] > 8) {
           w = w1[a];
           lds_write4(pa + (uint32_t)lane * 4u, pr1[a]);
           pk = pa + ko;
@@ -492,17 +503,19 @@ __global__ __launch_bounds__(1024) void union_attn_kernel(const UnionParams p) {
         kr = kr2;
         vr = vr2;
       };
+      const int ns = un[a] >> 1;
       int s = 0;
       if (a == 0) {
-        if (ns[0] > 0) next_step(0);
+        if (ns > 0) next_step(0);
         s = 1;
         // Past the end the last tile again, into the buffer no tile reads any more.
         stage(min(n + 1, ntiles - 1), lds0 + (bo ^ 65536u));
         load_list(n + 2, aft);
-        put_rows(nxt, half ^ (NB * 256u), nsn, krn, vrn);
+        put_rows(nxt, half ^ (NB * 256u), unn, krn, vrn);
       }
 #pragma unroll 1
-      for (; s < ns[a]; ++s) next_step(s);
+      for (; s < ns; ++s) next_step(s);
+      if (un[a] & 1) step(std::integral_constant<int, 1>{}, a, w, kr, vr, kx + bo, vx + bo);
     }
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0): this wave's copies of tile n + 1, its lists
@@ -510,7 +523,7 @@ __global__ __launch_bounds__(1024) void union_attn_kernel(const UnionParams p) {
     asm volatile("" ::: "memory");
 #pragma unroll
     for (int a = 0; a < NB; ++a) {
-      ns[a] = nsn[a];
+      un[a] = unn[a];
       kr0[a] = krn[a];
       vr0[a] = vrn[a];
     }
@@ -578,11 +591,12 @@ UnionLayout union_layout(int64_t B, int64_t T, int64_t S, int64_t H) {
   return L;
 }
 
-// Waves per workgroup and 16-query blocks per wave. One workgroup fits a CU's LDS, and its time
-// grows with its blocks plus a fixed part (the copies and barriers, about 6 blocks' worth), so a
-// launch takes about rounds x (blocks + 6): the pair with the smallest product. Two blocks a
-// wave halve the K and V traffic, which bounds long key ranges (87,936 keys: 12.5 ms, one
-// block 14.4); at 43,968 one block fills the last round better (4.6 against 4.7-4.85).
+// Waves per workgroup and 16-query blocks per wave. One workgroup fits a CU's LDS, so a launch
+// takes rounds x a workgroup's time: the blocks per SIMD (between the fullest SIMD's and the
+// mean; 15 % more each with three waves a SIMD to hide latency instead of four) plus about half a
+// block for the copies and barriers, fitted at 8 to 64 views. The shape with the smallest product. Two blocks a wave halve the
+// K and V traffic, which bounds long key ranges (87,936 keys: 11.8 ms, one block 14.5); at
+// 43,968 one block fills the last round better (4.34 against 4.5 ms).
 struct UnionShape {
   int waves, nb;
 };
@@ -590,9 +604,11 @@ UnionShape union_shape(int64_t nblocks, int64_t heads, int cus) {
   UnionShape best = {16, 1};
   double best_t = 1e300;
   for (int nb = 1; nb <= 2; ++nb)
-    for (int w = 16; w >= 8; --w) {
+    for (int w = 16; w >= 9; --w) {
       const int64_t wgs = (nblocks + w * nb - 1) / (w * nb) * heads;
-      const double t = (double)((wgs + cus - 1) / cus) * (w * nb + 6);
+      const int per_simd = (w + 3) / 4;
+      const double blocks = 0.5 * (per_simd + 0.25 * w) * nb * (per_simd == 4 ? 1.0 : 1.15);
+      const double t = (double)((wgs + cus - 1) / cus) * (blocks + 0.5);
       if (t < best_t) {
         best_t = t;
         best = {w, nb};

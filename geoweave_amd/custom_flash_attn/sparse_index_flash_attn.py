@@ -134,10 +134,11 @@ def _dense_fits(k: torch.Tensor, q_layout: str, seqlen_k: int, seqlen_q: int = 0
 
 # "auto" without attn_sum takes the union pass (gw_sparse_attn_fwd_union) in place of the dense
 # one where a query selects at most 1 / UNION_MIN_RATIO of the keys: sixteen queries then
-# select at most 62 % of them together. Measured in ms (16 heads, K = 1,024; dense, union): S / K
-# = 10.7 0.65, 0.75; 16.1 1.43, 1.39; 21.5 2.28, 1.92; 32.2 4.74, 3.42; 42.9 7.45, 4.6; 85.9 28.4, 12.5.
+# select at most two thirds of them together. Measured in ms (16 heads, K = 1,024; dense, union):
+# S / K = 10.7 0.64, 0.73; 13.4 0.95, 1.02; 14.8 1.09, 1.10; 16.1 1.40, 1.36; 21.5 2.26, 1.83;
+# 32.2 4.7, 3.2; 42.9 7.4, 4.34; 85.9 28.2, 11.8.
 # Beyond DENSE_MAX_RATIO the gather stays: it keeps P in fp32, both matrix-core passes in fp16.
-UNION_MIN_RATIO = 17
+UNION_MIN_RATIO = 15
 
 
 def _use_union(seqlen_k: int, num_kv: int, d: int, softmax_scale: float, return_attn: bool) -> bool:
