@@ -19,6 +19,7 @@
 //     out[i] = x[i] c - x[i+16] s,   out[i+16] = x[i+16] c + x[i] s
 //   (rope.py:120-152: x * cos + cat(-x2, x1) * sin with cos/sin = cat(t, t) tables).
 #include <algorithm>
+#include <type_traits>
 
 #include "gw_common.h"
 
@@ -49,6 +50,8 @@ struct GlueParams {
   uint16_t* ik_out;        // [rows, Hi, 64]
   uint16_t* iw_out;        // [rows, Hi]
   int64_t rows;
+  int v_off;               // casting kernels only: the v block, copied to v_out [rows, H, 64]
+  uint16_t* v_out;
 };
 
 // Eight lanes per head vector: lane j of a group holds dims [8j, 8j + 8) as one 16-byte
@@ -65,7 +68,7 @@ struct GlueVec {
   int head, out_heads, col;
   int norm;  // -1: none, 0: attention q, 1: attention k, 2: indexer k
   uint16_t* out;
-  bool live, gate;
+  bool live, gate, plain;  // plain: no norm, no rotation (v)
 };
 
 __device__ __forceinline__ GlueVec glue_vec(const GlueParams& p, uint32_t vid, uint32_t nvec, uint32_t slots) {
@@ -93,18 +96,35 @@ __device__ __forceinline__ GlueVec glue_vec(const GlueParams& p, uint32_t vid, u
     v.out = p.iq_out;
     v.out_heads = p.Hi;
     v.gate = true;  // the indexer gate of this head travels with its query vector
-  } else {
+  } else if (slot < 2 * p.H + 2 * p.Hi) {
     v.head = slot - 2 * p.H - p.Hi;
     v.col = p.ik_off + v.head * kGlueD;
     v.norm = p.ikn_w ? 2 : -1;
     v.out = p.ik_out;
     v.out_heads = p.Hi;
+  } else {  // casting kernels
+    v.head = slot - 2 * p.H - 2 * p.Hi;
+    v.col = p.v_off + v.head * kGlueD;
+    v.out = p.v_out;
+    v.out_heads = p.H;
+    v.plain = true;
   }
   return v;
 }
 
+// O: the element type of the outputs. Where it is not E (the score dtype), every value is rounded
+// to E and then to O, as a cast after the glue would, and v is copied along (a cast of each
+// tensor after the glue took 240 us of a 16-view layer's 2.9 ms).
 template <typename E>
+__device__ __forceinline__ float glue_round(float x) {
+  float lo, hi;
+  unpack2(E{}, pack1(E{}, x), lo, hi);
+  return lo;
+}
+
+template <typename E, typename O>
 __global__ __launch_bounds__(256) void dsa_glue_kernel(const GlueParams p) {
+  constexpr bool CAST = !std::is_same<E, O>::value;
   __shared__ float ln_s[3][2][kGlueD];  // (q, k, indexer k) x (weight, bias)
   __shared__ float rope_s[2][kGlueMaxRope * 16];
   const float* lnw[3] = {p.qn_w, p.kn_w, p.ikn_w};
@@ -125,7 +145,7 @@ __global__ __launch_bounds__(256) void dsa_glue_kernel(const GlueParams p) {
   const float* cos_t = rope_lds ? rope_s[0] : p.rope_cos;
   const float* sin_t = rope_lds ? rope_s[1] : p.rope_sin;
 
-  const uint32_t slots = 2 * p.H + 2 * p.Hi;
+  const uint32_t slots = (CAST ? 3 : 2) * p.H + 2 * p.Hi;
   const uint32_t nvec = (uint32_t)(p.rows * slots);
   const int lane = threadIdx.x & 63;
   const int j = lane & 7;  // 16-byte chunk of each vector
@@ -146,7 +166,12 @@ __global__ __launch_bounds__(256) void dsa_glue_kernel(const GlueParams p) {
       const int64_t row = v[u].row;
       float x[8];
       unpack8<E>(raw[u], x);
-      if (v[u].gate && j == 0) p.iw_out[row * p.Hi + v[u].head] = p.y[row * p.ldy + p.iw_off + v[u].head];
+      if (v[u].gate && j == 0) {
+        const uint16_t g = p.y[row * p.ldy + p.iw_off + v[u].head];
+        float gf, unused;
+        unpack2(E{}, (uint32_t)g, gf, unused);
+        p.iw_out[row * p.Hi + v[u].head] = CAST ? (uint16_t)pack1(O{}, gf) : g;
+      }
       if (v[u].norm >= 0) {  // uniform over the 8-lane group
         const float* g = &ln_s[v[u].norm][0][8 * j];
         const float* bta = &ln_s[v[u].norm][1][8 * j];
@@ -164,7 +189,7 @@ __global__ __launch_bounds__(256) void dsa_glue_kernel(const GlueParams p) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] = (x[e] - mean) * rstd * g[e] + bta[e];
       }
-      if (p.pos != nullptr) {
+      if (p.pos != nullptr && !(CAST && v[u].plain)) {  // uniform over the 8-lane group
         const int pp = min(max(p.pos[row * 2 + (j >> 2)], 0), p.rope_len - 1);  // y below dim 32, x above
         const float* c = cos_t + pp * 16 + 8 * (j & 1);
         const float* sn = sin_t + pp * 16 + 8 * (j & 1);
@@ -175,7 +200,11 @@ __global__ __launch_bounds__(256) void dsa_glue_kernel(const GlueParams p) {
           x[e] = x[e] * c[e] + sign * partner * sn[e];
         }
       }
-      *reinterpret_cast<uint4*>(v[u].out + (row * v[u].out_heads + v[u].head) * kGlueD + 8 * j) = pack8<E>(x);
+      if constexpr (CAST) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = glue_round<E>(x[e]);
+      }
+      *reinterpret_cast<uint4*>(v[u].out + (row * v[u].out_heads + v[u].head) * kGlueD + 8 * j) = pack8<O>(x);
     }
   }
 }
@@ -339,19 +368,22 @@ __global__ __launch_bounds__(64 * kLnReduceSums) void dsa_glue_ln_reduce_kernel(
 }  // namespace
 }  // namespace gw
 
-extern "C" int gw_dsa_glue_fwd(int dtype, const void* y, int64_t rows, int64_t ldy, int64_t q_off, int64_t k_off,
+namespace gw {
+namespace {
+
+int glue_fwd_impl(int dtype, int out_dtype, int64_t v_off, void* v_out, const void* y, int64_t rows, int64_t ldy, int64_t q_off, int64_t k_off,
                                int64_t iq_off, int64_t ik_off, int64_t iw_off, int64_t H, int64_t Hi, int64_t D,
                                const float* q_norm_w, const float* q_norm_b, const float* k_norm_w,
                                const float* k_norm_b, const float* idx_k_norm_w, const float* idx_k_norm_b,
                                float ln_eps, const int32_t* pos, const float* rope_cos, const float* rope_sin,
                                int64_t rope_len, void* q_out, void* k_out, void* idx_q_out, void* idx_k_out,
                                void* idx_w_out, void* stream) {
-  using namespace gw;
-  clear_error();
   GW_CHECK_ARG(dtype == GW_DTYPE_BF16 || dtype == GW_DTYPE_FP16, "unsupported dtype code %d", dtype);
   if (D != kGlueD) return set_error(GW_ERR_UNSUPPORTED, "head dim %lld not supported (64)", (long long)D);
   GW_CHECK_ARG(rows >= 0 && H >= 1 && Hi >= 0 && H <= 64 && Hi <= 64, "invalid sizes rows=%lld H=%lld Hi=%lld",
                (long long)rows, (long long)H, (long long)Hi);
+  const bool cast = out_dtype != dtype;
+  GW_CHECK_ARG(out_dtype == GW_DTYPE_BF16 || out_dtype == GW_DTYPE_FP16, "unsupported output dtype code %d", out_dtype);
   if (rows == 0) return GW_OK;
   GW_CHECK_ARG(y && q_out && k_out && (Hi == 0 || (idx_q_out && idx_k_out && idx_w_out)), "null tensor pointer");
   GW_CHECK_ARG(ldy % 8 == 0 && aligned16(y), "projection rows must be 16-byte aligned (ldy %% 8 == 0)");
@@ -369,6 +401,12 @@ extern "C" int gw_dsa_glue_fwd(int dtype, const void* y, int64_t rows, int64_t l
   GW_CHECK_ARG(aligned16(q_out) && aligned16(k_out) && aligned16(idx_q_out) && aligned16(idx_k_out),
                "outputs must be 16-byte aligned");  // null (Hi = 0) counts as aligned
   GW_CHECK_ARG(rows * (2 * H + 2 * Hi) < (1ll << 31) - 64, "rows x head vectors exceeds the 32-bit index range");
+  if (cast) {
+    GW_CHECK_ARG(v_out != nullptr && aligned16(v_out), "v_out must be a 16-byte aligned tensor");
+    GW_CHECK_ARG(v_off >= 0 && v_off % 8 == 0 && v_off + H * D <= ldy, "column block v at %lld must be 8-aligned and inside ldy=%lld",
+                 (long long)v_off, (long long)ldy);
+    GW_CHECK_ARG(rows * (3 * H + 2 * Hi) < (1ll << 31) - 64, "rows x head vectors exceeds the 32-bit index range");
+  }
   GlueParams p{};
   p.y = static_cast<const uint16_t*>(y);
   p.ldy = ldy;
@@ -396,16 +434,54 @@ extern "C" int gw_dsa_glue_fwd(int dtype, const void* y, int64_t rows, int64_t l
   p.ik_out = static_cast<uint16_t*>(idx_k_out);
   p.iw_out = static_cast<uint16_t*>(idx_w_out);
   p.rows = rows;
-  const int64_t vectors = rows * (2 * H + 2 * Hi);
+  p.v_off = (int)v_off;
+  p.v_out = static_cast<uint16_t*>(v_out);
+  const int64_t vectors = rows * ((cast ? 3 : 2) * H + 2 * Hi);
   const int64_t waves = (vectors + 8 * kGlueVecs - 1) / (8 * kGlueVecs);
   const dim3 grid((unsigned)std::min<int64_t>((waves + 3) / 4, 2048));
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (dtype == GW_DTYPE_BF16)
-    hipLaunchKernelGGL((dsa_glue_kernel<BF16>), grid, dim3(256), 0, st, p);
-  else
-    hipLaunchKernelGGL((dsa_glue_kernel<FP16>), grid, dim3(256), 0, st, p);
+  if (dtype == GW_DTYPE_BF16) {
+    if (cast)
+      hipLaunchKernelGGL((dsa_glue_kernel<BF16, FP16>), grid, dim3(256), 0, st, p);
+    else
+      hipLaunchKernelGGL((dsa_glue_kernel<BF16, BF16>), grid, dim3(256), 0, st, p);
+  } else {
+    if (cast)
+      hipLaunchKernelGGL((dsa_glue_kernel<FP16, BF16>), grid, dim3(256), 0, st, p);
+    else
+      hipLaunchKernelGGL((dsa_glue_kernel<FP16, FP16>), grid, dim3(256), 0, st, p);
+  }
   GW_HIP_LAUNCH_CHECK("dsa_glue_kernel");
   return GW_OK;
+}
+
+}  // namespace
+}  // namespace gw
+
+extern "C" int gw_dsa_glue_fwd(int dtype, const void* y, int64_t rows, int64_t ldy, int64_t q_off, int64_t k_off,
+                               int64_t iq_off, int64_t ik_off, int64_t iw_off, int64_t H, int64_t Hi, int64_t D,
+                               const float* q_norm_w, const float* q_norm_b, const float* k_norm_w,
+                               const float* k_norm_b, const float* idx_k_norm_w, const float* idx_k_norm_b,
+                               float ln_eps, const int32_t* pos, const float* rope_cos, const float* rope_sin,
+                               int64_t rope_len, void* q_out, void* k_out, void* idx_q_out, void* idx_k_out,
+                               void* idx_w_out, void* stream) {
+  gw::clear_error();
+  return gw::glue_fwd_impl(dtype, dtype, 0, nullptr, y, rows, ldy, q_off, k_off, iq_off, ik_off, iw_off, H, Hi, D, q_norm_w, q_norm_b, k_norm_w, k_norm_b,
+                            idx_k_norm_w, idx_k_norm_b, ln_eps, pos, rope_cos, rope_sin, rope_len, q_out, k_out, idx_q_out,
+                            idx_k_out, idx_w_out, stream);
+}
+
+extern "C" int gw_dsa_glue_fwd_cast(int dtype, int out_dtype, int64_t v_off, void* v_out, const void* y, int64_t rows, int64_t ldy, int64_t q_off, int64_t k_off,
+                               int64_t iq_off, int64_t ik_off, int64_t iw_off, int64_t H, int64_t Hi, int64_t D,
+                               const float* q_norm_w, const float* q_norm_b, const float* k_norm_w,
+                               const float* k_norm_b, const float* idx_k_norm_w, const float* idx_k_norm_b,
+                               float ln_eps, const int32_t* pos, const float* rope_cos, const float* rope_sin,
+                               int64_t rope_len, void* q_out, void* k_out, void* idx_q_out, void* idx_k_out,
+                               void* idx_w_out, void* stream) {
+  gw::clear_error();
+  return gw::glue_fwd_impl(dtype, out_dtype, v_off, v_out, y, rows, ldy, q_off, k_off, iq_off, ik_off, iw_off, H, Hi, D, q_norm_w, q_norm_b, k_norm_w, k_norm_b,
+                            idx_k_norm_w, idx_k_norm_b, ln_eps, pos, rope_cos, rope_sin, rope_len, q_out, k_out, idx_q_out,
+                            idx_k_out, idx_w_out, stream);
 }
 
 extern "C" size_t gw_dsa_glue_bwd_workspace_size(int64_t rows, int64_t H, int64_t Hi) {

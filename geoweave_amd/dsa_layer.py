@@ -159,9 +159,11 @@ def dsa_glue_forward(
     pos: Optional[torch.Tensor] = None,
     rope_base: float = 100.0,
     rope_len: Optional[int] = None,
+    out_dtype: Optional[torch.dtype] = None,
 ):
     """(q, k, v, idx_q, idx_k, idx_w) from the fused projection ``y [B, N, ldy]`` via
-    ``gw_dsa_glue_fwd``. q/k ``[B, N, H, 64]`` and idx_q/idx_k ``[B, N, Hi, 64]`` are new
+    ``gw_dsa_glue_fwd``, or, with an ``out_dtype`` other than y's (the other 16-bit type), cast
+    to it in the same pass (``gw_dsa_glue_fwd_cast``; v is then a tensor of its own). q/k ``[B, N, H, 64]`` and idx_q/idx_k ``[B, N, Hi, 64]`` are new
     contiguous tensors, idx_w ``[B, N, Hi]``; v is a strided view of ``y``. ``pos`` is
     ``[B, N, 2]`` (y, x) integer positions or None (no rope); ``rope_len`` is the table
     length (default ``max(pos) + 1`` like the reference, ``rope.py:190``, which reads it on
@@ -173,11 +175,12 @@ def dsa_glue_forward(
     B, N = y.shape[0], y.shape[1]
     H, Hi = layout.H, layout.Hi
     dev = y.device
-    q = torch.empty(B, N, H, 64, device=dev, dtype=y.dtype)
+    od = y.dtype if out_dtype is None else out_dtype
+    q = torch.empty(B, N, H, 64, device=dev, dtype=od)
     k = torch.empty_like(q)
-    iq = torch.empty(B, N, Hi, 64, device=dev, dtype=y.dtype) if Hi else None
+    iq = torch.empty(B, N, Hi, 64, device=dev, dtype=od) if Hi else None
     ik = torch.empty_like(iq) if Hi else None
-    iw = torch.empty(B, N, Hi, device=dev, dtype=y.dtype) if Hi else None
+    iw = torch.empty(B, N, Hi, device=dev, dtype=od) if Hi else None
     pos32 = cos = sin = None
     n_rope = 0
     if pos is not None:
@@ -187,18 +190,21 @@ def dsa_glue_forward(
         n_rope = int(rope_len) if rope_len is not None else int(pos32.max()) + 1
         cos, sin = rope2d_tables(n_rope, rope_base, dev)
     lib = _lib.load()
-    _lib.check(
-        lib.gw_dsa_glue_fwd(
-            _lib.dtype_code(y.dtype), y.data_ptr(), B * N, layout.ldy, layout.q_off, layout.k_off,
-            layout.iq_off, layout.ik_off, layout.iw_off, H, Hi, 64,
-            _lib.ptr(q_norm[0]), _lib.ptr(q_norm[1]), _lib.ptr(k_norm[0]), _lib.ptr(k_norm[1]),
-            _lib.ptr(idx_k_norm[0]), _lib.ptr(idx_k_norm[1]), float(ln_eps),
-            _lib.ptr(pos32), _lib.ptr(cos), _lib.ptr(sin), n_rope,
-            q.data_ptr(), k.data_ptr(), _lib.ptr(iq), _lib.ptr(ik), _lib.ptr(iw),
-            _lib.stream_handle(dev),
-        ),
-        "gw_dsa_glue_fwd",
+    args = (
+        y.data_ptr(), B * N, layout.ldy, layout.q_off, layout.k_off,
+        layout.iq_off, layout.ik_off, layout.iw_off, H, Hi, 64,
+        _lib.ptr(q_norm[0]), _lib.ptr(q_norm[1]), _lib.ptr(k_norm[0]), _lib.ptr(k_norm[1]),
+        _lib.ptr(idx_k_norm[0]), _lib.ptr(idx_k_norm[1]), float(ln_eps),
+        _lib.ptr(pos32), _lib.ptr(cos), _lib.ptr(sin), n_rope,
+        q.data_ptr(), k.data_ptr(), _lib.ptr(iq), _lib.ptr(ik), _lib.ptr(iw),
+        _lib.stream_handle(dev),
     )
+    if od != y.dtype:
+        v = torch.empty_like(q)
+        _lib.check(lib.gw_dsa_glue_fwd_cast(_lib.dtype_code(y.dtype), _lib.dtype_code(od), layout.v_off, v.data_ptr(),
+                                            *args), "gw_dsa_glue_fwd_cast")
+        return q, k, v, iq, ik, iw
+    _lib.check(lib.gw_dsa_glue_fwd(_lib.dtype_code(y.dtype), *args), "gw_dsa_glue_fwd")
     v = y[..., layout.v_off:layout.v_off + H * 64].view(B, N, H, 64)
     return q, k, v, iq, ik, iw
 
@@ -403,8 +409,11 @@ class SparseGlobalAttention(nn.Module):
         q, k, v, iq, ik, iw = dsa_glue_forward(
             y, self.layout, _ln_params(self.q_norm), _ln_params(self.k_norm), _ln_params(self.indexer.k_norm),
             self.q_norm.eps if isinstance(self.q_norm, nn.LayerNorm) else 1e-5,
-            pos if self.rope_base else None, self.rope_base or 100.0, rope_len)
-        q, k, v, iq, ik, iw = self._to_score_dtype(x.dtype, q, k, v, iq, ik, iw)
+            pos if self.rope_base else None, self.rope_base or 100.0, rope_len,
+            # a 16-bit score dtype is cast to in the same pass, float32 after it
+            self.score_dtype if self.score_dtype in (torch.float16, torch.bfloat16) else None)
+        if self.score_dtype == torch.float32:
+            q, k, v, iq, ik, iw = self._to_score_dtype(x.dtype, q, k, v, iq, ik, iw)
         kk = min(int(topk or self.topk), N)
         if query_chunk is not None and 0 < int(query_chunk) < N and topk_indices is None:
             o = sparse_attention_streaming(q, k, v, iq, ik, iw, kk, int(query_chunk), float(self.indexer.scale),

@@ -324,6 +324,20 @@ int gw_dsa_glue_fwd(int dtype, const void* y, int64_t rows, int64_t ldy, int64_t
                     void* idx_w_out, void* stream);
 
 /* ------------------------------------------------------------------------------------
+ * gw_dsa_glue_fwd with its outputs in out_dtype (the other 16-bit type: the reference's
+ * score_dtype cast, dsa_attention.py:4943-4948): every value rounded to dtype, then to out_dtype,
+ * and the v block [v_off, +H*64) of y cast to v_out [rows, H, 64] as well. Equal types: as
+ * gw_dsa_glue_fwd (v_off and v_out unused).
+ */
+int gw_dsa_glue_fwd_cast(int dtype, int out_dtype, int64_t v_off, void* v_out, const void* y, int64_t rows,
+                         int64_t ldy, int64_t q_off, int64_t k_off, int64_t iq_off, int64_t ik_off,
+                         int64_t iw_off, int64_t H, int64_t Hi, int64_t D, const float* q_norm_w,
+                         const float* q_norm_b, const float* k_norm_w, const float* k_norm_b,
+                         const float* idx_k_norm_w, const float* idx_k_norm_b, float ln_eps, const int32_t* pos,
+                         const float* rope_cos, const float* rope_sin, int64_t rope_len, void* q_out,
+                         void* k_out, void* idx_q_out, void* idx_k_out, void* idx_w_out, void* stream);
+
+/* ------------------------------------------------------------------------------------
  * DSA layer glue, backward (training through the layer).
  *
  * Gradient of gw_dsa_glue_fwd, i.e. of the reference's q_norm/k_norm + rope + cast glue
