@@ -141,6 +141,14 @@ def _dense_fits(k: torch.Tensor, q_layout: str, seqlen_k: int, seqlen_q: int = 0
 UNION_MIN_RATIO = 15
 
 
+# "auto" with attn_sum runs the pass without it and then the mass from its lse
+# (gw_sparse_attn_mass) where a query selects at least 1 / MASS_MAX_RATIO of the keys: the mass pass
+# recomputes every score (~ T·S), the dense pass with attn_sum stores the selected ones of
+# every head (~ T·K). Measured in ms (16 heads, K = 1,024; stored, recomputed): S / K = 1.3
+# 0.22, 0.15; 2.7 0.31, 0.18; 5.4 0.59, 0.40; 9.4 1.25, 0.99; 10.7 1.33, 1.25; 16.1 2.83, 2.86.
+MASS_MAX_RATIO = 10
+
+
 def _use_union(seqlen_k: int, num_kv: int, d: int, softmax_scale: float, return_attn: bool) -> bool:
     if FORWARD_PATH not in ("auto", "union") or d != 64 or return_attn:
         return False
@@ -214,25 +222,38 @@ def _flash_attn_forward(
         float(softmax_scale),
     )
     stream = _lib.stream_handle(q.device)
-    if kl_logits is None:
-        kl_args = (None, 0, 0, 0, 0.0, None)
-    else:
+    kl_args = no_kl = (None, 0, 0, 0, 0.0, None)
+    if kl_logits is not None:
         code = _lib.GW_DTYPE_FP32 if kl_logits.dtype == torch.float32 else _lib.dtype_code(kl_logits.dtype)
         kl_args = (kl_logits.data_ptr(), code, kl_logits.stride(0), kl_logits.stride(1), float(kl_eps),
                    kl_row_loss.data_ptr())
-    if _use_union(seqlen_k, num_kv, d, softmax_scale, return_attn):
+    dense = (_use_dense(seqlen_k, num_kv, nheads, d, softmax_scale) and _dense_fits(k, q_layout, seqlen_k, seqlen_q)
+             and (attn_sum is None or num_kv <= DENSE_ATTN_SUM_MAX_K))
+    separate_mass = (FORWARD_PATH == "auto" and dense and attn_sum is not None and nheads <= 64
+                     and seqlen_k <= MASS_MAX_RATIO * num_kv
+                     and _bthd_strides(q, q_layout)[1] < DENSE_MAX_K_ROW_STRIDE)
+    union = _use_union(seqlen_k, num_kv, d, softmax_scale, attn_sum is not None and not separate_mass)
+    if union:
         ws_bytes = int(lib.gw_sparse_attn_fwd_union_workspace_size(batch, seqlen_q, seqlen_k, nheads, d, num_kv))
         ws = torch.empty(max(ws_bytes, 1), device=q.device, dtype=torch.uint8)
         rc = lib.gw_sparse_attn_fwd_union(*common[:13], *common[14:], ws.data_ptr(), ws_bytes, stream)
         _lib.check(rc, "gw_sparse_attn_fwd_union")
-        return o, attn_sum, lse, softmax_scale
-    if (_use_dense(seqlen_k, num_kv, nheads, d, softmax_scale) and _dense_fits(k, q_layout, seqlen_k, seqlen_q)
-            and (attn_sum is None or num_kv <= DENSE_ATTN_SUM_MAX_K)):
+    elif dense:
+        want_attn = attn_sum is not None and not separate_mass
         dense_bytes = int(lib.gw_sparse_attn_fwd_dense_workspace_size(batch, seqlen_q, seqlen_k, nheads, d, num_kv,
-                                                                      int(attn_sum is not None)))
-        dws = torch.empty(max(dense_bytes, 1), device=q.device, dtype=torch.uint8)
-        rc = lib.gw_sparse_attn_fwd_dense(*common, *kl_args, dws.data_ptr(), dense_bytes, stream)
+                                                                      int(want_attn)))
+        ws = torch.empty(max(dense_bytes, 1), device=q.device, dtype=torch.uint8)
+        rc = lib.gw_sparse_attn_fwd_dense(*common[:13], common[13] if want_attn else None, *common[14:],
+                                          *(kl_args if want_attn else no_kl), ws.data_ptr(), dense_bytes, stream)
         _lib.check(rc, "gw_sparse_attn_fwd_dense")
+    if separate_mass:
+        del ws
+        ws_bytes = int(lib.gw_sparse_attn_mass_workspace_size(batch, seqlen_q, seqlen_k, nheads, d, num_kv))
+        ws = torch.empty(max(ws_bytes, 1), device=q.device, dtype=torch.uint8)
+        rc = lib.gw_sparse_attn_mass(*common[:5], *common[7:10], *common[12:14], *common[14:], *kl_args,
+                                     ws.data_ptr(), ws_bytes, stream)
+        _lib.check(rc, "gw_sparse_attn_mass")
+    if union or dense:
         return o, attn_sum, lse, softmax_scale
     ws, ws_bytes = None, 0
     if attn_sum is not None:

@@ -565,6 +565,29 @@ int gw_sparse_attn_fwd_union(int dtype,
                              void* stream);
 
 /* ------------------------------------------------------------------------------------
+ * Attention mass of the selected keys from a forward's lse: attn_sum[b, t, j] =
+ * sum_h exp(softmax_scale q.k - lse[b, t, h]) at the key of position j (0 outside [0, S)), the
+ * attn_sum of gw_sparse_attn_fwd; with logits also the KL row losses of gw_sparse_attn_fwd_kl
+ * (row_loss fp32 [B * T]). lse: fp32 [B, T, H], natural log, of the same q, k and positions.
+ * Recomputes the scores of every (query, key) pair on the matrix cores, summing over heads in
+ * registers. Needs D = 64, K <= 1024 and Q and K token strides below 2^23 elements; otherwise
+ * GW_ERR_UNSUPPORTED. Workspace: gw_sparse_attn_mass_workspace_size(B, T, S, H, D, K) bytes,
+ * 16-byte aligned: the sums of a chunk of queries, at most 256 MiB or 512 rows.
+ * ------------------------------------------------------------------------------------ */
+size_t gw_sparse_attn_mass_workspace_size(int64_t B, int64_t T, int64_t S, int64_t H, int64_t D, int64_t K);
+int gw_sparse_attn_mass(int dtype,
+                        const void* q, const int64_t* q_strides,
+                        const void* k, const int64_t* k_strides,
+                        const int32_t* kv_pos, int64_t pos_stride_b, int64_t pos_stride_t,
+                        const float* lse, float* attn_sum,
+                        int64_t B, int64_t T, int64_t S, int64_t H, int64_t D, int64_t K,
+                        float softmax_scale,
+                        const void* logits, int logits_dtype, int64_t logits_stride_b,
+                        int64_t logits_stride_t, float eps, float* row_loss,
+                        void* workspace, size_t workspace_bytes,
+                        void* stream);
+
+/* ------------------------------------------------------------------------------------
  * Sparse-index attention backward as masked dense passes: the same gradients as
  * gw_sparse_attn_bwd without an attn_sum gradient (dq, dk, dv up to fp32 summation order and
  * the rounding of P and dS to the input type for their matrix products), computed on the
