@@ -145,8 +145,9 @@ UNION_MIN_RATIO = 15
 # (gw_sparse_attn_mass) where a query selects at least 1 / MASS_MAX_RATIO of the keys: the mass pass
 # recomputes every score (~ T·S), the dense pass with attn_sum stores the selected ones of
 # every head (~ T·K). Measured in ms (16 heads, K = 1,024; stored, recomputed): S / K = 1.3
-# 0.22, 0.15; 2.7 0.31, 0.18; 5.4 0.59, 0.40; 9.4 1.25, 0.99; 10.7 1.33, 1.25; 16.1 2.83, 2.86.
-MASS_MAX_RATIO = 10
+# 0.22, 0.15; 2.7 0.34, 0.19; 5.4 0.67, 0.40; 9.4 1.41, 0.99; 10.7 1.52, 1.23; 16.1 2.91, 2.73;
+# 32.2 8.46, 9.21. The two vary by a tenth between runs, so the line lies below where they meet.
+MASS_MAX_RATIO = 12
 
 
 def _use_union(seqlen_k: int, num_kv: int, d: int, softmax_scale: float, return_attn: bool) -> bool:
@@ -232,7 +233,10 @@ def _flash_attn_forward(
     separate_mass = (FORWARD_PATH == "auto" and dense and attn_sum is not None and nheads <= 64
                      and seqlen_k <= MASS_MAX_RATIO * num_kv
                      and _bthd_strides(q, q_layout)[1] < DENSE_MAX_K_ROW_STRIDE)
-    union = _use_union(seqlen_k, num_kv, d, softmax_scale, attn_sum is not None and not separate_mass)
+    # "auto" takes the union pass only in place of the dense one: a call beyond the dense limits
+    # stays with the gather kernel.
+    union = ((FORWARD_PATH == "union" or dense)
+             and _use_union(seqlen_k, num_kv, d, softmax_scale, attn_sum is not None and not separate_mass))
     if union:
         ws_bytes = int(lib.gw_sparse_attn_fwd_union_workspace_size(batch, seqlen_q, seqlen_k, nheads, d, num_kv))
         ws = torch.empty(max(ws_bytes, 1), device=q.device, dtype=torch.uint8)
