@@ -15,9 +15,11 @@ Printed: ONE JSON line. ``value`` = indexer ms + attention-forward ms per layer 
 better). ``roofline`` = the attention forward (the dominant call) against the roofline of
 what it executes, timed live with HIP events on the stream the kernels run on: for the
 masked dense pass the bf16 MFMA roofline on its flops (every (query, key) product,
-4*B*T*S*H*D), for the gather kernel the HBM roofline on the gathered K/V bytes.
+4*B*T*S*H*D), for the union pass the same roofline on the selected products alone
+(4*B*T*K*H*D; it executes those of the keys that any of 16 queries selected), for the gather
+kernel the HBM roofline on the gathered K/V bytes.
 ``attn_effective_gathered_bandwidth`` = the sparse formulation's gathered bytes over the
-same time (a rate, not a roofline, for the dense pass). ``roofline_indexer`` = the indexer
+same time (a rate, not a roofline, for the dense and union passes). ``roofline_indexer`` = the indexer
 against the bf16 MFMA roofline. ``cpu_baseline`` = the fp32 CPU oracle (the restatement of
 the reference's torch backend) on a fixed sample of query rows of the same layer (median of
 3 passes, scaled to the full layer), plus config C1 timed in full (median of 3 runs) beside
@@ -47,6 +49,15 @@ def attn_fwd_algorithmic_bytes(B, T, H, D, K, elt=2):
     """Gathered K and V rows (K per query, shared by the H heads) + q read + o write +
     int32 positions: B*T*K*H*D*2*elt + 2*B*T*H*D*elt + 4*B*T*K."""
     return B * T * K * H * D * 2 * elt + 2 * B * T * H * D * elt + 4 * B * T * K
+
+
+def attn_fwd_path(T, K, H, D, scale=0.125):
+    """The attention forward without attn_sum that the dispatch takes for S = T keys."""
+    from geoweave_amd.custom_flash_attn import sparse_index_flash_attn as sifa
+
+    if not sifa._use_dense(T, K, H, D, scale) and sifa.FORWARD_PATH != "union":
+        return "gather"
+    return "union" if sifa._use_union(T, K, D, scale, False) else "dense"
 
 
 def attn_fwd_dense_flops(B, T, S, H, D):
@@ -210,9 +221,7 @@ def long_context_c3(steps: int = 5, warmup: int = 2, views: int = 64, topk: int 
     att_ms = statistics.mean(e[1].elapsed_time(e[2]) for e in evs)
     B, T, H, D = q.shape
     att_bytes = attn_fwd_algorithmic_bytes(B, T, H, D, topk)
-    from geoweave_amd.custom_flash_attn import sparse_index_flash_attn as sifa
-
-    attn_path = "dense" if sifa._use_dense(T, topk, H, D, 0.125) else "gather"
+    attn_path = attn_fwd_path(T, topk, H, D)
 
     # The query-chunked stream (dsa_attention.py:1017-1283): same work, the indices and the
     # indexer workspace live per chunk of 16384 queries. Peak memory above the inputs.
@@ -619,7 +628,7 @@ def main() -> int:
     ap.add_argument("--no-sd", action="store_true", help="skip the approximate (source-downsample) top-k timing")
     ap.add_argument("--attn-path", choices=("auto", "dense", "gather"), default="auto",
                     help="attention forward without attn_sum: the masked dense pass, the gather kernel, "
-                         "or the automatic choice (dense when S <= 96 K)")
+                         "or the automatic choice (dense below 15 K keys, union up to 96 K)")
     ap.add_argument("--calibrate-copy", action="store_true",
                     help="also run 3 plain device copies of 1 GiB (reference kernel for rocprofv3 "
                          "FETCH_SIZE / WRITE_SIZE scaling)")
@@ -696,11 +705,11 @@ def main() -> int:
     att_avg = statistics.mean(att_ms)
     idx_avg = statistics.mean(idx_ms)
     att_gbs = att_bytes / (att_avg * 1e-3) / 1e9
-    dense_flops = attn_fwd_dense_flops(B, T, T, H, D)
-    dense_tflops = dense_flops / (att_avg * 1e-3) / 1e12
+    attn_path = attn_fwd_path(T, Kk, H, D)
+    attn_flops = attn_fwd_dense_flops(B, T, Kk if attn_path == "union" else T, H, D)
+    attn_tflops = attn_flops / (att_avg * 1e-3) / 1e12
     idx_tflops = idx_flops / (idx_avg * 1e-3) / 1e12
-    dense_used = sifa._use_dense(T, Kk, H, D)
-    prof_name = f"dense_attn_fwd_S{views}_pmc.md" if dense_used else f"sparse_attn_fwd_S{views}_pmc.md"
+    prof_name = {"dense": "dense", "union": "union", "gather": "sparse"}[attn_path] + f"_attn_fwd_S{views}_pmc.md"
     traffic = read_traffic_summary(REPO / "profiles" / prof_name)
 
     extra = {}
@@ -738,20 +747,23 @@ def main() -> int:
         },
         "indexer_ms": round(idx_avg, 3),
         "attn_fwd_ms": round(att_avg, 3),
-        "attn_path": "dense" if dense_used else "gather",
-        # The roofline of what runs: the masked dense pass is bound by the matrix cores on
-        # the flops it executes; the gather kernel by HBM on the bytes it gathers.
+        "attn_path": attn_path,
+        # The roofline of what runs: the masked dense pass against the matrix cores on
+        # the flops it executes, the union pass on the selected products alone (it is bound by
+        # the instructions around them), the gather kernel against HBM on the bytes it gathers.
         "roofline": ({
-            "kernel": "dense_attn_kernel (one attention call: + dense_mask_kernel, dense_vmax_kernel, "
-                      "dense_vt_kernel)",
+            "kernel": ("union_attn_kernel (one attention call: + union_lists_kernel, union_tiles_kernel, "
+                       "dense_vmax_kernel)" if attn_path == "union" else
+                       "dense_attn_kernel (one attention call: + dense_mask_kernel, dense_vmax_kernel, "
+                       "dense_vt_kernel)"),
             "bound": "mfma",
-            "achieved": round(dense_tflops, 2),
+            "achieved": round(attn_tflops, 2),
             "peak": MFMA_BF16_PEAK_TFLOPS,
             "unit": "TFLOP/s",
-            "frac": round(dense_tflops / MFMA_BF16_PEAK_TFLOPS, 4),
+            "frac": round(attn_tflops / MFMA_BF16_PEAK_TFLOPS, 4),
             "traffic": traffic,
-            "algorithmic_flops": dense_flops,
-        } if dense_used else {
+            "algorithmic_flops": attn_flops,
+        } if attn_path != "gather" else {
             "kernel": "sparse_attn_fwd_kernel",
             "bound": "hbm",
             "achieved": round(att_gbs, 1),
@@ -763,7 +775,7 @@ def main() -> int:
         }),
         # The sparse formulation's bytes (the selected K/V rows the reference gathers) over
         # the call's time: an effective rate of the whole attention, not a roofline of the
-        # dense pass (which does not move these bytes).
+        # dense or union pass (which do not move these bytes).
         "attn_effective_gathered_bandwidth": {
             "gathered_bytes": att_bytes,
             "achieved": round(att_gbs, 1),
