@@ -141,3 +141,21 @@ def test_routes(gpu_device):
         o, lse = _run(q, k, v, pos, path="auto")
         og, lg = _run(q, k, v, pos, path="gather")
         assert (o - og).norm() <= 2 * REL[torch.bfloat16] * og.norm() and (lse - lg).abs().max() < 1e-4
+
+
+@pytest.mark.parametrize("limit,value", [("DENSE_MAX_S", 100), ("DENSE_MAX_T", 16), ("DENSE_MAX_K_ROW_STRIDE", 64)])
+def test_calls_beyond_the_dense_limits_stay_with_the_gather(gpu_device, monkeypatch, limit, value):
+    # With the dense limits lowered below the call, "auto" gives the gather kernel's bits, not the union's.
+    print(f"[union] {limit}", flush=True)
+    g = torch.Generator().manual_seed(11)
+    q, k, v = (torch.randn(1, n, 2, 64, generator=g).bfloat16().cuda() for n in (40, 640, 640))
+    pos = torch.rand(1, 40, 640, generator=g).topk(32, dim=-1).indices.to(torch.int32).cuda()
+
+    def run(path):
+        monkeypatch.setattr(sifa, "FORWARD_PATH", path)
+        return sifa._flash_attn_forward(q, k, v, pos, softmax_scale=0.125, return_attn=False)[0]
+
+    gather, union = run("gather"), run("union")
+    assert torch.equal(run("auto"), union) and not torch.equal(gather, union)
+    monkeypatch.setattr(sifa, limit, value)
+    assert torch.equal(run("auto"), gather)
