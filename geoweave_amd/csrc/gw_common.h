@@ -265,4 +265,41 @@ __device__ __forceinline__ void buffer_load16_lds(const char* base, uint32_t off
                                            (int)off, 0, 0, 0);
 }
 
+// The same 16 bytes a lane from memory to LDS, issued through inline asm: the compiler does not
+// see that the instruction writes LDS, so it neither waits for the copy before the next LDS read
+// nor orders it. The caller waits (s_waitcnt vmcnt(0)) before the barrier after which the data is
+// read. M0 carries the wave's LDS byte address and is restored afterwards.
+// The hardware does not interlock a scalar write of M0 with a load to LDS (one wait state is
+// due), nor a vector write of a scalar register (the base, by v_readfirstlane) with a memory
+// instruction that reads it (five): inside an asm string the wait states are the string's own,
+// so an s_nop stands before the load (together with the two scalar moves at least five).
+//
+// lds_dma16: a 64-bit address per lane. lds_dma16_s: a wave-uniform base and a 32-bit offset per
+// lane (no 64-bit address arithmetic per load).
+__device__ __forceinline__ void lds_dma16(const void* src, uint32_t lds) {
+  uint32_t saved;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(saved)
+      : "v"(src), "s"(__builtin_amdgcn_readfirstlane(lds))
+      : "memory");
+}
+__device__ __forceinline__ void lds_dma16_s(const void* base, uint32_t off, uint32_t lds) {
+  const uint64_t bu = reinterpret_cast<uint64_t>(uniform_ptr(static_cast<const char*>(base)));
+  uint32_t saved;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %3\n\t"
+      "s_nop 2\n\t"
+      "global_load_lds_dwordx4 %1, %2\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(saved)
+      : "v"(off), "s"(bu), "s"(__builtin_amdgcn_readfirstlane(lds))
+      : "memory");
+}
+
 }  // namespace gw

@@ -282,41 +282,10 @@ __device__ __forceinline__ int sweep_key(int i, const ScoreParams& p) {
 // (32 consecutive key rows at one logical chunk) then hit 16 distinct 16-byte bank groups
 // per 16 lanes (8 for HI = 1), one LDS pass per 256 bytes.
 //
-// The loads are issued through inline asm, so the compiler does not see instructions that
-// write LDS behind its back: otherwise it cannot tell that a prefetch into one stage buffer
-// does not alias the operand reads of the other, and waits for the prefetch (vmcnt(0))
-// before the first read. The kernel waits for the loads itself (vmcnt(0) before the stage
-// barrier). M0 carries the wave's LDS destination and is restored after each load.
-__device__ __forceinline__ void lds_dma16(const void* src, const void* lds_dst) {
-  const uint32_t lds = (uint32_t)(uintptr_t)lds_dst;
-  uint32_t saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %2\n\t"
-      "global_load_lds_dwordx4 %1, off\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "v"(src), "s"(__builtin_amdgcn_readfirstlane(lds))
-      : "memory");
-}
-
-// The same load from a wave-uniform base (an SGPR pair) plus a 32-bit per-lane offset: no
-// 64-bit address arithmetic per load.
-__device__ __forceinline__ void lds_dma16_s(const void* base, uint32_t off, const void* lds_dst) {
-  const uint32_t lds = (uint32_t)(uintptr_t)lds_dst;
-  const uint64_t b = reinterpret_cast<uintptr_t>(base);
-  const uint64_t bu = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) << 32) |
-                      (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
-  uint32_t saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %3\n\t"
-      "global_load_lds_dwordx4 %1, %2\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "v"(off), "s"(bu), "s"(__builtin_amdgcn_readfirstlane(lds))
-      : "memory");
-}
+// The loads are inline asm (lds_dma16), or the compiler, which cannot tell that a prefetch into
+// one stage buffer does not alias the operand reads of the other, would wait for the prefetch
+// (vmcnt(0)) before the first read. The kernel waits for the loads itself, before the stage
+// barrier.
 
 // Workgroup shape of the score kernel, by the bytes of a key row (HI heads of 64 elements):
 // NW waves of 32 queries share every key tile (a key tile read from L2 serves NW * 32
@@ -483,7 +452,7 @@ __global__ __launch_bounds__((ScoreShape<row_bytes<E, HI>()>::THREADS),
       // Full stage of consecutive keys: uniform base + lane offset + i * NW KB.
       const char* kbase = static_cast<const char*>(p.k) + ((int64_t)b * S + kb) * ROW_BYTES;
 #pragma unroll
-      for (int i = 0; i < LOADS; ++i) lds_dma16_s(kbase, voffs[i], &ktile[(i * NW + wave) * 1024]);
+      for (int i = 0; i < LOADS; ++i) lds_dma16_s(kbase, voffs[i], (uint32_t)(uintptr_t)&ktile[(i * NW + wave) * 1024]);
     } else {
       // Sample keys or the last stage: rows past the end re-read the last valid key.
 #pragma unroll
@@ -492,7 +461,7 @@ __global__ __launch_bounds__((ScoreShape<row_bytes<E, HI>()>::THREADS),
         const int key = sweep_key<SAMPLE>(kb + kl, p);
         const int lc = lc0 ^ ((i * RPI) & SWZ);
         const char* src = static_cast<const char*>(p.k) + ((int64_t)b * S + key) * ROW_BYTES + lc * 16;
-        lds_dma16(src, &ktile[(i * NW + wave) * 1024]);
+        lds_dma16(src, (uint32_t)(uintptr_t)&ktile[(i * NW + wave) * 1024]);
       }
     }
 #pragma unroll

@@ -46,18 +46,6 @@ struct MassParams {
   float scale_log2;
 };
 
-// Direct global-to-LDS copy of 1 KB: lane i moves the 16 bytes at base + off to lds + 16 i. Inline
-// asm: the compiler would wait for it before the next LDS read.
-__device__ __forceinline__ void mass_dma(const char* base, uint32_t off, uint32_t lds) {
-  const uint64_t bu = reinterpret_cast<uint64_t>(uniform_ptr(base));
-  uint32_t saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "v"(off), "s"(bu), "s"(__builtin_amdgcn_readfirstlane(lds))
-      : "memory");
-}
-
 template <typename E>
 __global__ __launch_bounds__(kMWaves * 64) void attn_mass_kernel(const MassParams p) {
   // Two K tiles (a head's and the next one's), then each wave's 32 query rows of one head.
@@ -97,8 +85,8 @@ __global__ __launch_bounds__(kMWaves * 64) void attn_mass_kernel(const MassParam
   float l2n;
   auto stage = [&](int h, uint32_t kto) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) mass_dma(qbase + (int64_t)h * p.qsh * 2, qoff[i], qs0 + i * 1024);
-    mass_dma(kbase + (int64_t)h * p.ksh * 2, koff, kto + (uint32_t)wave * 1024u);
+    for (int i = 0; i < 4; ++i) lds_dma16_s(qbase + (int64_t)h * p.qsh * 2, qoff[i], qs0 + i * 1024);
+    lds_dma16_s(kbase + (int64_t)h * p.ksh * 2, koff, kto + (uint32_t)wave * 1024u);
     l2n = lse[h];
   };
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));

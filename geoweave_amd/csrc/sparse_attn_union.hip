@@ -277,18 +277,6 @@ __device__ __forceinline__ uint2 lds_read_tr(uint32_t a) {
   return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4f16(reinterpret_cast<lds_h4*>((uintptr_t)a)));
 }
 
-// Direct global-to-LDS copy of 1 KB: lane i moves 16 bytes to lds + 16 i. Inline asm, so that the
-// compiler does not wait for it before the next LDS read (the kernel waits before the barrier).
-__device__ __forceinline__ void union_dma(const uint8_t* base, uint32_t off, uint32_t lds) {
-  const uint64_t bu = reinterpret_cast<uint64_t>(uniform_ptr(reinterpret_cast<const char*>(base)));
-  uint32_t saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "v"(off), "s"(bu), "s"(__builtin_amdgcn_readfirstlane(lds))
-      : "memory");
-}
-
 // -inf where bit 7 of byte j of w is set, else 0 (one sign-extended byte select and mask).
 __device__ __forceinline__ float select_bias16(uint32_t w, int j) {
   return __uint_as_float((uint32_t)(int32_t)(int8_t)(w >> (8 * j)) & 0xFF800000u);
@@ -339,7 +327,7 @@ __global__ __launch_bounds__(1024) void union_attn_kernel(const UnionParams p) {
     const uint8_t* tb = src + (int64_t)n * kUTileBytes;
     for (int s0 = wave; s0 < kUTileBytes / 1024; s0 += nw) {
       const uint32_t s = (uint32_t)(s0 + rot) & (kUTileBytes / 1024 - 1);
-      union_dma(tb + s * 1024, (uint32_t)lane * 16u, to + s * 1024);
+      lds_dma16_s(tb + s * 1024, (uint32_t)lane * 16u, to + s * 1024);
     }
   };
   const uint32_t kx = lds0 + ((uint32_t)g << 4);
