@@ -404,7 +404,9 @@ __global__ __launch_bounds__((ScoreShape<row_bytes<E, HI>()>::THREADS),
   const int stride = SAMPLE ? 0 : kSubTotal / nsplit;
   int2* const lbase = SAMPLE ? nullptr : p.cand + (((int64_t)b * T + q0) * nsplit + split) * stride;
   const uint32_t wstart = (uint32_t)(col * nsplit * stride) * 8u;
-  const uint32_t wend = wstart + (uint32_t)p.cap * 8u;  // first byte past the list's slots
+  // First byte past the list's slots. A lane past the last query has no list: its scores (of a
+  // zero query) are NaN where a key or gate is not finite, and a NaN can carry the mark.
+  const uint32_t wend = row_ok ? wstart + (uint32_t)p.cap * 8u : wstart;
   uint32_t woff = wstart;
 
   // Loader geometry: load i of this thread fills LDS bytes [(i*NW + wave)*1024 + 16*lane, +16),
