@@ -773,6 +773,10 @@ struct SelectParams {
   float tau0;
 };
 
+// The key of a candidate, never 0, which marks an empty slot: f2key is 0 for one NaN (all bits
+// set), and a row of nothing else would leave the bisection an empty range that never ends.
+__device__ __forceinline__ uint32_t live_key(float v) { return max(f2key(v), 1u); }
+
 // Number of set bits of a wave mask below this lane.
 __device__ __forceinline__ int lanes_below(uint64_t m) {
   return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
@@ -821,7 +825,8 @@ __device__ __forceinline__ bool row_lists(const SelectParams& p, int64_t row, Ro
 // ROWS: the candidates are all keys, their scores read from a score row instead of lists (short
 // key sets, see Plan::rows_all). The entries keep the lists' order: entry 64 m + l of a row is
 // the key that the filter's lane half l / 32 holds as element l % 16 of tile l % 32 / 16 of
-// stage m (stages of 64 keys; of 32: half l % 32 / 16, stage 2 m + l / 32), and keys that the filter would not mark (score - inf, or NaN) stay out.
+// stage m (stages of 64 keys; of 32: half l % 32 / 16, stage 2 m + l / 32), and keys that the
+// filter would not mark (score -inf, or a NaN whose sign bit is clear) stay out.
 template <typename E, int KS, bool ROWS>
 __global__ __launch_bounds__(256) void indexer_select_kernel(const SelectParams p) {
   __shared__ uint32_t cbuf[4][kCompactKeys];
@@ -847,7 +852,7 @@ __global__ __launch_bounds__(256) void indexer_select_kernel(const SelectParams 
       const float v = __uint_as_float(kv[m]);
       const bool live = ky[m] < p.S && (int32_t)__float_as_uint(p.tau0 - v) < 0;
       total += __popcll(__ballot(live));
-      kv[m] = live ? f2key(v) : 0u;
+      kv[m] = live ? live_key(v) : 0u;
     }
   } else {
     bad = row_lists(p, row, rl);
@@ -900,13 +905,12 @@ __global__ __launch_bounds__(256) void indexer_select_kernel(const SelectParams 
     if (m0 < nch) {
 #pragma unroll
       for (int m = m0; m < m0 + 8; ++m)
-        if (m * 64 + lane < total) kv[m] = f2key(__uint_as_float(kv[m]));
+        if (m * 64 + lane < total) kv[m] = live_key(__uint_as_float(kv[m]));
     }
   }
   }
   // Key range of the live slots: empty slots hold 0, which kv - 1 wraps to the maximum (the
   // + 1 comes after the wave minimum, so a lane without live slots does not wrap back to 0).
-  // Candidates passed a >= comparison and are never NaN, so no live key is 0.
 #pragma unroll
   for (int m = 0; m < KS; ++m) {
     lmin = min(lmin, kv[m] - 1u);
