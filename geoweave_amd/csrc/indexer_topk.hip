@@ -444,8 +444,8 @@ __global__ __launch_bounds__((ScoreShape<row_bytes<E, HI>()>::THREADS),
   // Gate values travel as raw 16-bit patterns until wstore converts them at the end of the
   // stage: converting at load time would make the wave wait (vmcnt) for the key tile
   // loads issued just before. Keys past the end: K rows are loaded from the last valid key
-  // (harmless), and the gate is NaN (FILTER: the mark clears keys past the end)
-  // or 0 (SAMPLE: not stored).
+  // (harmless), and the gate is NaN (FILTER: the mark clears keys past the end; SAMPLE: not
+  // stored). An fp32 gate of this pattern is a NaN itself.
   constexpr uint32_t kNoGate = 0xFFFFFFFFu;
   uint32_t wraw[WLOADS];
   auto gload = [&](int kb, uint8_t* ktile) {
@@ -483,8 +483,7 @@ __global__ __launch_bounds__((ScoreShape<row_bytes<E, HI>()>::THREADS),
     for (int i = 0; i < WLOADS; ++i) {
       const int c = tid + THREADS * i;
       if (c < WVALS) {
-        const float wv = wraw[i] == kNoGate ? (SAMPLE ? 0.f : __builtin_nanf(""))
-                                            : to_f32(E{}, wraw[i]) * p.scale;
+        const float wv = wraw[i] == kNoGate ? __builtin_nanf("") : to_f32(E{}, wraw[i]) * p.scale;
         wtile[(c % HI) * BN + c / HI] = wv;
       }
     }
@@ -826,7 +825,7 @@ __device__ __forceinline__ bool row_lists(const SelectParams& p, int64_t row, Ro
 // key sets, see Plan::rows_all). The entries keep the lists' order: entry 64 m + l of a row is
 // the key that the filter's lane half l / 32 holds as element l % 16 of tile l % 32 / 16 of
 // stage m (stages of 64 keys; of 32: half l % 32 / 16, stage 2 m + l / 32), and keys that the
-// filter would not mark (score -inf, or a NaN whose sign bit is clear) stay out.
+// filter would not mark (score -inf, or a NaN with the sign bit set) stay out.
 template <typename E, int KS, bool ROWS>
 __global__ __launch_bounds__(256) void indexer_select_kernel(const SelectParams p) {
   __shared__ uint32_t cbuf[4][kCompactKeys];

@@ -26,3 +26,19 @@ def test_rows_of_nan_scores(gpu_device, every, S, flags, bits):
     # the rows without a NaN select as without the mask
     assert torch.equal(order[:, 1::2], plain.sort(-1).values[:, 1::2])
     assert torch.equal(scores.sort(-1).values[:, 1::2], plain_scores.sort(-1).values[:, 1::2])
+
+
+def test_nan_gate_of_all_bits(gpu_device):
+    # The pattern that stands for "no gate" inside the kernel, as a gate of the input: a NaN score
+    # on every path, not a score of 0.
+    print("[nan scores] gate of all bits", flush=True)
+    g = torch.Generator().manual_seed(1)
+    q, k = (torch.randn(1, n, 2, 64, generator=g).cuda() for n in (40, 700))
+    w = -(1 + 0.5 * torch.rand(1, 700, 2, generator=g)).cuda()  # other scores are not above 0
+    w[0, ::9] = torch.tensor([-1], dtype=torch.int32).view(torch.float32).cuda()
+    rows = sti.indexer_topk_forward(q, k, w, None, 100, 0.125)
+    lists = sti.indexer_topk_forward(q, k, w, None, 100, 0.125, flags=sti.FLAG_TAU_MINUS_INF)
+    torch.cuda.synchronize()
+    assert torch.equal(rows[0], lists[0])
+    assert torch.equal(rows[1].view(torch.int32), lists[1].view(torch.int32))
+    assert torch.equal(rows[1].isnan(), rows[0] % 9 == 0)
