@@ -140,9 +140,16 @@ __global__ __launch_bounds__(kMWaves * 64) void attn_mass_kernel(const MassParam
 }
 
 struct MassGatherParams {
+  const uint16_t* q;  // q, k and lse: for rows with an empty head
+  const uint16_t* k;
+  const float* lse;
+  int64_t qsb, qst, qsh;
+  int64_t ksb, kss, ksh;
+  int in_fp16, H;
+  float scale_log2;
   const int32_t* pos;
   int64_t psb, pst;
-  const float* a;
+  float* a;
   float* attn_sum;  // [B, T, K]
   const void* logits;
   int logits_dt;
@@ -169,6 +176,37 @@ __device__ __forceinline__ float mass_wave_max(float x) {
   return x;
 }
 
+// A head without weight in row t (lse = -inf: no score of a valid key above -inf) adds nothing to
+// the row's sums, whatever its scores are; the matrix kernel has added exp2(score + inf). The
+// wave sums the selected keys of such a row again over the other heads. Rare, and here because
+// a test of each weight in the matrix kernel costs it the registers of its fourth wave (5,496
+// keys: the forward with the mass 373 -> 642 us).
+__device__ __forceinline__ void mass_empty_heads(const MassGatherParams& p, int64_t t, const int32_t* prow, float* arow,
+                                                 int lane) {
+  const float* lse = p.lse + ((int64_t)p.b * p.T + t) * p.H;
+  bool empty = false;
+  for (int h = lane; h < p.H; h += 64) empty |= lse[h] == -INFINITY;
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(empty) == 0ull, 1)) return;
+#pragma unroll 1
+  for (int j = lane; j < p.K; j += 64) {
+    const int s = prow[j];
+    if ((uint32_t)s >= (uint32_t)p.S) continue;
+    float sum = 0.f;
+#pragma unroll 1
+    for (int h = 0; h < p.H; ++h) {
+      if (lse[h] == -INFINITY) continue;
+      const uint16_t* qr = p.q + p.b * p.qsb + t * p.qst + h * p.qsh;
+      const uint16_t* kr = p.k + p.b * p.ksb + (int64_t)s * p.kss + h * p.ksh;
+      float d = 0.f;
+#pragma unroll 1
+      for (int i = 0; i < 64; ++i) d = fmaf(in_to_float(p.in_fp16, qr[i]), in_to_float(p.in_fp16, kr[i]), d);
+      sum += fexp2(fmaf(d, p.scale_log2, -lse[h] * kDLog2e));
+    }
+    arow[s] = sum;
+  }
+  __threadfence_block();  // the stores before the wave's own loads of the row
+}
+
 // One wave per query row: the selected values of its matrix row (0 for positions outside [0, S)),
 // and with KL the row's loss from them.
 template <int R, bool KL>
@@ -178,7 +216,8 @@ __global__ __launch_bounds__(256) void attn_mass_gather_kernel(const MassGatherP
   if (row >= p.rows) return;  // whole wave; no barriers below
   const int64_t t = p.t0 + row;
   const int32_t* prow = p.pos + p.b * p.psb + t * p.pst;
-  const float* arow = p.a + (int64_t)row * p.Spad;
+  float* arow = p.a + (int64_t)row * p.Spad;
+  mass_empty_heads(p, t, prow, arow, lane);
   float* out = p.attn_sum + ((int64_t)p.b * p.T + t) * p.K;
   float av[R], zv[R];
   float sa = 0.f, mz = -INFINITY;
@@ -302,6 +341,14 @@ extern "C" int gw_sparse_attn_mass(int dtype, const void* q, const int64_t* q_st
   p.H = (int)H;
   p.scale_log2 = softmax_scale * kDLog2e;
   MassGatherParams g;
+  g.q = p.q;
+  g.k = p.k;
+  g.lse = lse;
+  g.qsb = p.qsb; g.qst = p.qst; g.qsh = p.qsh;
+  g.ksb = p.ksb; g.kss = p.kss; g.ksh = p.ksh;
+  g.in_fp16 = dtype == GW_DTYPE_FP16 ? 1 : 0;
+  g.H = p.H;
+  g.scale_log2 = p.scale_log2;
   g.pos = kv_pos;
   g.psb = pos_stride_b;
   g.pst = pos_stride_t;

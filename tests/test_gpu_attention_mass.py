@@ -70,3 +70,25 @@ def test_mass_of_repeated_positions_and_nonfinite_keys(gpu_device):
     k[1, 299], v[1, 299] = float("nan"), float("inf")  # a row that no query selected
     a = _attn(q, k, v, pos)
     assert ((a - ra).abs() <= 1e-5 * ra + 1e-7).all()
+
+
+@pytest.mark.parametrize("case", ["keys of -inf", "scores beyond fp32", "no valid key"])
+def test_mass_of_heads_without_weight(gpu_device, case, monkeypatch):
+    # Every selected score of a head is -inf: its lse is -inf, it adds nothing (the gather kernel's
+    # result, bit for bit where no other head adds).
+    print(f"[mass] {case}", flush=True)
+    q, k, v, pos = _case(1, 70, 200, 3, 30, torch.bfloat16, 23)
+    q = q.abs() + 1
+    if case == "keys of -inf":
+        k[:, :, 1] = -float("inf")
+    elif case == "scores beyond fp32":
+        q, k = q * 1e19, -(k.abs() + 1)
+        k[:, :, 1] *= 3e19
+        q[:, :, [0, 2]] *= 1e-19
+    else:
+        pos[:, ::2] = -1
+    a = _attn(q, k, v, pos)
+    monkeypatch.setattr(sifa, "FORWARD_PATH", "gather")
+    g = _attn(q, k, v, pos)
+    assert torch.isfinite(g).all() and torch.isfinite(a).all()
+    assert ((a - g).abs() <= 1e-5 * g + 1e-7).all()
