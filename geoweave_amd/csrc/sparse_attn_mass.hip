@@ -41,8 +41,9 @@ struct MassParams {
   float* a;          // [rows of the chunk][Spad]
   int64_t qsb, qst, qsh;
   int64_t ksb, kss, ksh;
-  int b, t0, rows;   // batch element, first query and queries of the chunk
-  int T, S, Spad, H, ngroup;
+  int g0, ngroup;    // the chunk's groups of kMRows queries: [g0, g0 + ngroup)
+  int gpb;           // groups per batch element: group g is queries [kMRows (g % gpb), ...) of element g / gpb
+  int T, S, Spad, H;
   float scale_log2;
 };
 
@@ -54,10 +55,12 @@ __global__ __launch_bounds__(kMWaves * 64) void attn_mass_kernel(const MassParam
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 31, half = lane >> 5;
   const int grp = blockIdx.x % p.ngroup, k0 = (blockIdx.x / p.ngroup) * kMKeys;
+  const int b = (p.g0 + grp) / p.gpb, t0 = (p.g0 + grp) % p.gpb * kMRows;
+  const int rows = min(kMRows, p.T - t0);
   const float sl2 = p.scale_log2;
-  const int row0 = grp * kMRows + wave * 32;  // this wave's first row of the chunk
-  const bool ok = row0 + col < p.rows;
-  const float* lse = p.lse + ((int64_t)p.b * p.T + p.t0 + (ok ? row0 + col : 0)) * p.H;
+  const int row0 = wave * 32;  // this wave's first row of the group
+  const bool ok = row0 + col < rows;
+  const float* lse = p.lse + ((int64_t)b * p.T + t0 + (ok ? row0 + col : 0)) * p.H;
   f32x16 acc[4];
 #pragma unroll
   for (int st = 0; st < 4; ++st)
@@ -71,16 +74,16 @@ __global__ __launch_bounds__(kMWaves * 64) void attn_mass_kernel(const MassParam
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)kt;
   const uint32_t qs0 = lds0 + 2 * kMKeys * 128 + (uint32_t)wave * 4096u;
   const uint32_t kss_b = (uint32_t)p.kss * 2u, qst_b = (uint32_t)p.qst * 2u;
-  const int qfirst = min(row0, p.rows - 1);
-  const char* kbase = reinterpret_cast<const char*>(p.k + p.b * p.ksb + (int64_t)k0 * p.kss);
-  const char* qbase = reinterpret_cast<const char*>(p.q + p.b * p.qsb + (int64_t)(p.t0 + qfirst) * p.qst);
+  const int qfirst = min(row0, rows - 1);
+  const char* kbase = reinterpret_cast<const char*>(p.k + b * p.ksb + (int64_t)k0 * p.kss);
+  const char* qbase = reinterpret_cast<const char*>(p.q + b * p.qsb + (int64_t)(t0 + qfirst) * p.qst);
   const int kR = wave * 8 + (lane >> 3);
   const uint32_t koff = __umul24((uint32_t)min(kR, p.S - 1 - k0), kss_b) + (uint32_t)(((lane & 7) ^ swz(kR)) << 4);
   uint32_t qoff[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int R = i * 8 + (lane >> 3);
-    qoff[i] = __umul24((uint32_t)(min(row0 + R, p.rows - 1) - qfirst), qst_b) + (uint32_t)(((lane & 7) ^ swz(R)) << 4);
+    qoff[i] = __umul24((uint32_t)(min(row0 + R, rows - 1) - qfirst), qst_b) + (uint32_t)(((lane & 7) ^ swz(R)) << 4);
   }
   float l2n;
   auto stage = [&](int h, uint32_t kto) __attribute__((always_inline)) {
@@ -130,7 +133,7 @@ __global__ __launch_bounds__(kMWaves * 64) void attn_mass_kernel(const MassParam
     asm volatile("" ::: "memory");
   }
   if (!ok) return;
-  float* row = p.a + (int64_t)(row0 + col) * p.Spad + k0 + 4 * half;
+  float* row = p.a + ((int64_t)grp * kMRows + row0 + col) * p.Spad + k0 + 4 * half;
 #pragma unroll
   for (int st = 0; st < 4; ++st)
 #pragma unroll
@@ -156,7 +159,7 @@ struct MassGatherParams {
   int64_t lsb, lst;
   float kl_eps;
   float* row_loss;
-  int b, t0, rows, T, S, Spad, K;
+  int g0, ngroup, gpb, T, S, Spad, K;
 };
 
 __device__ __forceinline__ float mass_load(int dt, const void* base, int64_t i) {
@@ -181,9 +184,9 @@ __device__ __forceinline__ float mass_wave_max(float x) {
 // wave sums the selected keys of such a row again over the other heads. Rare, and here because
 // a test of each weight in the matrix kernel costs it the registers of its fourth wave (5,496
 // keys: the forward with the mass 373 -> 642 us).
-__device__ __forceinline__ void mass_empty_heads(const MassGatherParams& p, int64_t t, const int32_t* prow, float* arow,
-                                                 int lane) {
-  const float* lse = p.lse + ((int64_t)p.b * p.T + t) * p.H;
+__device__ __forceinline__ void mass_empty_heads(const MassGatherParams& p, int b, int64_t t, const int32_t* prow,
+                                                 float* arow, int lane) {
+  const float* lse = p.lse + ((int64_t)b * p.T + t) * p.H;
   bool empty = false;
   for (int h = lane; h < p.H; h += 64) empty |= lse[h] == -INFINITY;
   if (__builtin_expect(__builtin_amdgcn_ballot_w64(empty) == 0ull, 1)) return;
@@ -195,8 +198,8 @@ __device__ __forceinline__ void mass_empty_heads(const MassGatherParams& p, int6
 #pragma unroll 1
     for (int h = 0; h < p.H; ++h) {
       if (lse[h] == -INFINITY) continue;
-      const uint16_t* qr = p.q + p.b * p.qsb + t * p.qst + h * p.qsh;
-      const uint16_t* kr = p.k + p.b * p.ksb + (int64_t)s * p.kss + h * p.ksh;
+      const uint16_t* qr = p.q + b * p.qsb + t * p.qst + h * p.qsh;
+      const uint16_t* kr = p.k + b * p.ksb + (int64_t)s * p.kss + h * p.ksh;
       float d = 0.f;
 #pragma unroll 1
       for (int i = 0; i < 64; ++i) d = fmaf(in_to_float(p.in_fp16, qr[i]), in_to_float(p.in_fp16, kr[i]), d);
@@ -212,13 +215,15 @@ __device__ __forceinline__ void mass_empty_heads(const MassGatherParams& p, int6
 template <int R, bool KL>
 __global__ __launch_bounds__(256) void attn_mass_gather_kernel(const MassGatherParams p) {
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
-  if (row >= p.rows) return;  // whole wave; no barriers below
-  const int64_t t = p.t0 + row;
-  const int32_t* prow = p.pos + p.b * p.psb + t * p.pst;
-  float* arow = p.a + (int64_t)row * p.Spad;
-  mass_empty_heads(p, t, prow, arow, lane);
-  float* out = p.attn_sum + ((int64_t)p.b * p.T + t) * p.K;
+  const int64_t row = (int64_t)blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+  const int grp = p.g0 + (int)(row / kMRows);
+  const int b = grp / p.gpb;
+  const int64_t t = (int64_t)(grp % p.gpb) * kMRows + row % kMRows;
+  if (t >= p.T) return;  // whole wave; no barriers below
+  const int32_t* prow = p.pos + b * p.psb + t * p.pst;
+  float* arow = p.a + row * p.Spad;
+  mass_empty_heads(p, b, t, prow, arow, lane);
+  float* out = p.attn_sum + ((int64_t)b * p.T + t) * p.K;
   float av[R], zv[R];
   float sa = 0.f, mz = -INFINITY;
   int ps[R];
@@ -233,7 +238,7 @@ __global__ __launch_bounds__(256) void attn_mass_gather_kernel(const MassGatherP
     if (j < p.K) {
       out[j] = av[i];
       if constexpr (KL) {
-        zv[i] = mass_load(p.logits_dt, p.logits, p.b * p.lsb + t * p.lst + j);
+        zv[i] = mass_load(p.logits_dt, p.logits, b * p.lsb + t * p.lst + j);
         sa += av[i];
         mz = fmaxf(mz, zv[i]);
       }
@@ -258,13 +263,13 @@ __global__ __launch_bounds__(256) void attn_mass_gather_kernel(const MassGatherP
       }
     }
     loss = mass_wave_sum(loss);
-    if (lane == 0) p.row_loss[(int64_t)p.b * p.T + t] = loss;
+    if (lane == 0) p.row_loss[(int64_t)b * p.T + t] = loss;
   }
 }
 
 template <bool KL>
 void launch_gather(const MassGatherParams& g, hipStream_t st) {
-  const dim3 grid((unsigned)((g.rows + 3) / 4));
+  const dim3 grid((unsigned)(g.ngroup * (kMRows / 4)));
   if (g.K <= 64)
     hipLaunchKernelGGL((attn_mass_gather_kernel<1, KL>), grid, dim3(256), 0, st, g);
   else if (g.K <= 256)
@@ -275,12 +280,20 @@ void launch_gather(const MassGatherParams& g, hipStream_t st) {
     hipLaunchKernelGGL((attn_mass_gather_kernel<16, KL>), grid, dim3(256), 0, st, g);
 }
 
-// Queries per chunk: whole workgroups, their matrix within kMChunkBytes (one workgroup at least).
-int64_t mass_chunk(int64_t T, int64_t S) {
-  const int64_t spad = (S + kMKeys - 1) / kMKeys * kMKeys;
-  const int64_t fit = kMChunkBytes / (spad * 4) / kMRows * kMRows;
-  const int64_t all = (T + kMRows - 1) / kMRows * kMRows;
-  return fit < kMRows ? kMRows : fit < all ? fit : all;
+// Groups of kMRows queries per chunk: those of all batch elements in one order, so that a chunk of
+// several small elements is one launch, their matrix within kMChunkBytes (one group at least).
+struct MassChunks {
+  int64_t gpb, groups, chunk;  // groups per batch element, in all, and per chunk
+  int64_t spad;
+};
+MassChunks mass_chunks(int64_t B, int64_t T, int64_t S) {
+  MassChunks c;
+  c.spad = (S + kMKeys - 1) / kMKeys * kMKeys;
+  c.gpb = (T + kMRows - 1) / kMRows;
+  c.groups = B * c.gpb;
+  const int64_t fit = kMChunkBytes / (c.spad * 4 * kMRows);
+  c.chunk = fit < 1 ? 1 : fit < c.groups ? fit : c.groups;
+  return c;
 }
 
 }  // namespace
@@ -288,7 +301,8 @@ int64_t mass_chunk(int64_t T, int64_t S) {
 
 extern "C" size_t gw_sparse_attn_mass_workspace_size(int64_t B, int64_t T, int64_t S, int64_t H, int64_t D, int64_t K) {
   if (B <= 0 || T <= 0 || S <= 0 || H <= 0 || K <= 0 || D != 64) return 0;
-  return (size_t)(gw::mass_chunk(T, S) * ((S + gw::kMKeys - 1) / gw::kMKeys * gw::kMKeys) * 4);
+  const gw::MassChunks c = gw::mass_chunks(B, T, S);
+  return (size_t)(c.chunk * gw::kMRows * c.spad * 4);
 }
 
 extern "C" int gw_sparse_attn_mass(int dtype, const void* q, const int64_t* q_strides, const void* k,
@@ -315,7 +329,8 @@ extern "C" int gw_sparse_attn_mass(int dtype, const void* q, const int64_t* q_st
   if (k_strides[1] < 0 || k_strides[1] >= (1ll << 23) || q_strides[1] < 0 || q_strides[1] >= (1ll << 23))
     return set_error(GW_ERR_UNSUPPORTED, "the mass pass needs Q and K token strides below 2^23 elements, got %lld, %lld",
                      (long long)q_strides[1], (long long)k_strides[1]);
-  GW_CHECK_ARG(B <= 65535 && T < (1ll << 31) - 65536 && S < (1ll << 30), "size exceeds the grid range");
+  GW_CHECK_ARG(B <= 65535 && T < (1ll << 31) - 65536 && S < (1ll << 30) && B * ((T + kMRows - 1) / kMRows) < (1ll << 31),
+               "size exceeds the grid range");
   const bool kl = logits != nullptr;
   if (kl) {
     GW_CHECK_ARG(row_loss != nullptr, "null row_loss pointer");
@@ -327,7 +342,7 @@ extern "C" int gw_sparse_attn_mass(int dtype, const void* q, const int64_t* q_st
   GW_CHECK_ARG(workspace != nullptr && workspace_bytes >= need && aligned16(workspace),
                "the mass pass needs a 16-byte aligned %zu-byte workspace, got %zu", need, workspace_bytes);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int64_t chunk = mass_chunk(T, S);
+  const MassChunks c = mass_chunks(B, T, S);
   MassParams p;
   p.q = static_cast<const uint16_t*>(q);
   p.k = static_cast<const uint16_t*>(k);
@@ -337,7 +352,8 @@ extern "C" int gw_sparse_attn_mass(int dtype, const void* q, const int64_t* q_st
   p.ksb = k_strides[0]; p.kss = k_strides[1]; p.ksh = k_strides[2];
   p.T = (int)T;
   p.S = (int)S;
-  p.Spad = (int)((S + kMKeys - 1) / kMKeys * kMKeys);
+  p.Spad = (int)c.spad;
+  p.gpb = (int)c.gpb;
   p.H = (int)H;
   p.scale_log2 = softmax_scale * kDLog2e;
   MassGatherParams g;
@@ -363,25 +379,22 @@ extern "C" int gw_sparse_attn_mass(int dtype, const void* q, const int64_t* q_st
   g.T = p.T;
   g.S = p.S;
   g.Spad = p.Spad;
+  g.gpb = p.gpb;
   g.K = (int)K;
-  for (int64_t b = 0; b < B; ++b)
-    for (int64_t t0 = 0; t0 < T; t0 += chunk) {
-      p.b = g.b = (int)b;
-      p.t0 = g.t0 = (int)t0;
-      p.rows = g.rows = (int)(T - t0 < chunk ? T - t0 : chunk);
-      p.ngroup = (p.rows + kMRows - 1) / kMRows;
-      const int64_t wgs = (int64_t)p.ngroup * (p.Spad / kMKeys);
-      GW_CHECK_ARG(wgs < (1ll << 31), "size exceeds the grid range");
-      if (dtype == GW_DTYPE_BF16)
-        hipLaunchKernelGGL((attn_mass_kernel<BF16>), dim3((unsigned)wgs), dim3(kMWaves * 64), 0, st, p);
-      else
-        hipLaunchKernelGGL((attn_mass_kernel<FP16>), dim3((unsigned)wgs), dim3(kMWaves * 64), 0, st, p);
-      GW_HIP_LAUNCH_CHECK("attn_mass_kernel launch");
-      if (kl)
-        launch_gather<true>(g, st);
-      else
-        launch_gather<false>(g, st);
-      GW_HIP_LAUNCH_CHECK("attn_mass_gather_kernel launch");
-    }
+  for (int64_t g0 = 0; g0 < c.groups; g0 += c.chunk) {
+    p.g0 = g.g0 = (int)g0;
+    p.ngroup = g.ngroup = (int)(c.groups - g0 < c.chunk ? c.groups - g0 : c.chunk);
+    const int64_t wgs = (int64_t)p.ngroup * (p.Spad / kMKeys);
+    if (dtype == GW_DTYPE_BF16)
+      hipLaunchKernelGGL((attn_mass_kernel<BF16>), dim3((unsigned)wgs), dim3(kMWaves * 64), 0, st, p);
+    else
+      hipLaunchKernelGGL((attn_mass_kernel<FP16>), dim3((unsigned)wgs), dim3(kMWaves * 64), 0, st, p);
+    GW_HIP_LAUNCH_CHECK("attn_mass_kernel launch");
+    if (kl)
+      launch_gather<true>(g, st);
+    else
+      launch_gather<false>(g, st);
+    GW_HIP_LAUNCH_CHECK("attn_mass_gather_kernel launch");
+  }
   return GW_OK;
 }

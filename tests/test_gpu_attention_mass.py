@@ -46,7 +46,7 @@ def test_mass_edges(gpu_device, B, T, S, H, K, dtype):
 
 
 def test_mass_in_chunks_with_kl(gpu_device, monkeypatch):
-    # 60,000 keys: 512 rows a chunk of the score matrix's 256 MiB leave three chunks of 1,400 rows.
+    # 60,000 keys: the score matrix's 256 MiB hold 1,024 rows a chunk, so chunks of 1,024, 1,024 and 552.
     print("[mass] chunks, KL", flush=True)
     monkeypatch.setattr(sifa, "MASS_MAX_RATIO", 1 << 20)
     g = torch.Generator().manual_seed(3)
@@ -92,3 +92,19 @@ def test_mass_of_heads_without_weight(gpu_device, case, monkeypatch):
     g = _attn(q, k, v, pos)
     assert torch.isfinite(g).all() and torch.isfinite(a).all()
     assert ((a - g).abs() <= 1e-5 * g + 1e-7).all()
+
+
+def test_mass_chunks_across_batch_elements(gpu_device, monkeypatch):
+    # Three groups of 512 queries an element and 60,000 keys: chunks of two groups, the second of them
+    # with the last queries of element 0 and the first of element 1. Then six small elements in one.
+    monkeypatch.setattr(sifa, "MASS_MAX_RATIO", 1 << 20)
+    for B, T, S, K in ((3, 1100, 60000, 40), (6, 33, 200, 64)):
+        print(f"[mass] {B} elements of {T} queries", flush=True)
+        g = torch.Generator().manual_seed(S)
+        q, k, v = (torch.randn(B, n, 2, 64, generator=g).bfloat16() for n in (T, S, S))
+        pos = ((torch.randint(0, S, (B, T, 1), generator=g) + torch.arange(K).view(1, 1, K) * 7919) % S).to(torch.int32)
+        z = torch.randn(B, T, K, generator=g)
+        _, a, loss = sparse_attention_kl_loss(q.cuda(), k.cuda(), v.cuda(), pos.cuda(), z.cuda(), 1e-6, 0.125)
+        _, ra, _ = oatt.sparse_attention(q.float(), k.float(), v.float(), pos, 0.125)
+        assert ((a.cpu() - ra).abs() <= 1e-5 * ra + 1e-7).all()
+        assert abs(float(loss) - float(okl.kl_loss(ra, z, 1e-6))) <= 1e-5
