@@ -142,12 +142,25 @@ UNION_MIN_RATIO = 15
 
 
 # "auto" with attn_sum runs the pass without it and then the mass from its lse
-# (gw_sparse_attn_mass) where a query selects at least 1 / MASS_MAX_RATIO of the keys: the mass pass
-# recomputes every score (~ T·S), the dense pass with attn_sum stores the selected ones of
-# every head (~ T·K). Measured in ms (16 heads, K = 1,024; stored, recomputed): S / K = 1.3
-# 0.22, 0.15; 2.7 0.34, 0.19; 5.4 0.67, 0.40; 9.4 1.41, 0.99; 10.7 1.52, 1.23; 16.1 2.91, 2.73;
-# 32.2 8.46, 9.21. The two vary by a tenth between runs, so the line lies below where they meet.
+# (gw_sparse_attn_mass) where that is the faster of the two: the mass pass recomputes every score
+# (~ T·S), the dense pass with attn_sum stores the selected ones of every head (~ T·K) and sums
+# them.
+# - Where a query selects few of the keys the stores win. The line lies at S = 12 K for few query
+#   rows and nearer 9 K for many, where the recomputed scores fill the chip several times.
+#   Measured as recomputed / stored time, 16 heads: one element, K = 1,024, S / K = 9 0.80, 11
+#   0.93, 12 0.98; two 9 0.89, 10 0.95, 12 1.05; eight, K = 512, 9 0.99, 10 1.03, 11 1.07.
+# - A workgroup of the mass pass takes the heads one after another, about 4 us each, however
+#   small the call, while the stores and their sum grow with S and K. Recomputed / stored, 16 heads:
+#   S x K = 700 x 512 0.98, 1,536 x 384 0.91, 2,112 x 192 1.02, 1,024 x 256 1.16, 300 x 128 1.6;
+#   4 heads: 1,408 x 128 0.92, 512 x 128 1.03; 1 head: 256 x 64 1.00, 83 x 64 1.10.
 MASS_MAX_RATIO = 12
+MASS_MAX_RATIO_MANY = 9
+MASS_MIN_WORK = 26_000  # S * K per head
+
+
+def _use_mass(batch: int, seqlen_q: int, seqlen_k: int, nheads: int, num_kv: int) -> bool:
+    ratio = MASS_MAX_RATIO_MANY + (MASS_MAX_RATIO - MASS_MAX_RATIO_MANY) * min(1.0, seqlen_k / (batch * seqlen_q))
+    return seqlen_k <= ratio * num_kv and seqlen_k * num_kv >= MASS_MIN_WORK * nheads
 
 
 def _use_union(seqlen_k: int, num_kv: int, d: int, softmax_scale: float, return_attn: bool) -> bool:
@@ -231,7 +244,7 @@ def _flash_attn_forward(
     dense = (_use_dense(seqlen_k, num_kv, nheads, d, softmax_scale) and _dense_fits(k, q_layout, seqlen_k, seqlen_q)
              and (attn_sum is None or num_kv <= DENSE_ATTN_SUM_MAX_K))
     separate_mass = (FORWARD_PATH == "auto" and dense and attn_sum is not None and nheads <= 64
-                     and seqlen_k <= MASS_MAX_RATIO * num_kv
+                     and _use_mass(batch, seqlen_q, seqlen_k, nheads, num_kv)
                      and _bthd_strides(q, q_layout)[1] < DENSE_MAX_K_ROW_STRIDE)
     # "auto" takes the union pass only in place of the dense one: a call beyond the dense limits
     # stays with the gather kernel.
