@@ -159,3 +159,57 @@ def test_calls_beyond_the_dense_limits_stay_with_the_gather(gpu_device, monkeypa
     assert torch.equal(run("auto"), union) and not torch.equal(gather, union)
     monkeypatch.setattr(sifa, limit, value)
     assert torch.equal(run("auto"), gather)
+
+
+def _against_gather(q, k, v, pos, rows):
+    """Every (row, head) of the union pass against the gather kernel, and the given rows against the oracle."""
+    o, lse = _run(q, k, v, pos)
+    og, lg = _run(q, k, v, pos, path="gather")
+    rel = REL[q.dtype] + (2.0 ** -9 if q.dtype == torch.bfloat16 else 2.0 ** -12)
+    assert (o - og).norm() <= rel * og.norm()
+    # a head's 64 values: their errors' norm within 8 times the mean's (a wrong tile, list or row gives O(1))
+    assert ((o - og).norm(dim=-1) <= 8 * rel * og.norm(dim=-1) + 1e-6).all()
+    ok = torch.isfinite(lg)  # -inf: rows without a valid key
+    assert torch.equal(lse[~ok], lg[~ok]) and (lse[ok] - lg[ok]).abs().max() <= 1e-4
+    _check(q[:, rows], k, v, pos[:, rows], o[:, rows], lse[:, rows])
+
+
+# Queries for which the launch takes 9 to 16 waves of one or two 16-query blocks (16 heads, 256 CUs).
+SHAPES = {(9, 1): 301, (10, 1): 2330, (11, 1): 2590, (12, 1): 2853, (13, 1): 3100, (14, 1): 3361, (15, 1): 3610,
+          (16, 1): 3870, (9, 2): 4130, (10, 2): 4650, (11, 2): 5131, (12, 2): 5650, (13, 2): 6170, (14, 2): 6693,
+          (15, 2): 7200, (16, 2): 7727}
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_launch_shapes(gpu_device, shape):
+    # Tile 0 holds most keys (more than eight units a block), tiles 1 and 3 a few, tile 2 none, tile 4
+    # the ragged end; some rows without valid keys, one with a repeated position in a later block.
+    T = SHAPES[shape]
+    dtype = torch.float16 if shape[0] % 2 else torch.bfloat16
+    print(f"[union] {shape[0]} waves of {shape[1]} blocks, T={T} {dtype}", flush=True)
+    S, K = 1033, 40
+    q, k, v = _inputs(1, T, S, 16, dtype, T)
+    pos = torch.cat([_positions(1, T, S, 28, 1, 0, 256), _positions(1, T, S, 5, 2, 256, 512),
+                     _positions(1, T, S, 4, 3, 768, 1024), _positions(1, T, S, 3, 4, 1024, S)], -1)
+    pos = pos[..., torch.randperm(K, generator=torch.Generator().manual_seed(5))]
+    pos[:, 5::97, :] = -1
+    pos[:, 3::11, 20:] = -1
+    pos[0, T - 3, 7] = pos[0, T - 3, 6]
+    rows = sorted(set(range(0, T, 83)) | set(range(T - 40, T)) | {15, 16, 31, 32})
+    _against_gather(q, k, v, pos, rows)
+
+
+@pytest.mark.parametrize("S", [32769, 34816, 34817, 70000])
+def test_long_key_ranges(gpu_device, S):
+    # 129 and 136 tiles: the most that one pass over the positions holds; 137 and 274: two and three passes.
+    print(f"[union] S={S}", flush=True)
+    T, K = 70, 400
+    q, k, v = _inputs(1, T, S, 2, torch.bfloat16, S)
+    edge = (S + 255) // 256 // (1 + (S > 34816) + (S > 69632)) * 256  # about the first pass's end
+    near = _positions(1, T, S, 100, 8, max(0, edge - 700), min(S, edge + 700))
+    far = _positions(1, T, S, K - 100, 9, 0, max(0, edge - 700))
+    pos = torch.cat([near, far], -1)
+    pos[0, 20, 3] = pos[0, 20, 50]  # near the line
+    pos[0, 50, 3] = S - 1
+    pos[0, 50, 4] = S - 1
+    _against_gather(q, k, v, pos, list(range(0, T, 3)))
