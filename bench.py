@@ -51,13 +51,13 @@ def attn_fwd_algorithmic_bytes(B, T, H, D, K, elt=2):
     return B * T * K * H * D * 2 * elt + 2 * B * T * H * D * elt + 4 * B * T * K
 
 
-def attn_fwd_path(T, K, H, D, scale=0.125):
+def attn_fwd_path(B, T, K, H, D, scale=0.125):
     """The attention forward without attn_sum that the dispatch takes for S = T keys."""
     from geoweave_amd.custom_flash_attn import sparse_index_flash_attn as sifa
 
     if not sifa._use_dense(T, K, H, D, scale) and sifa.FORWARD_PATH != "union":
         return "gather"
-    return "union" if sifa._use_union(T, K, D, scale, False) else "dense"
+    return "union" if sifa._use_union(B, T, T, K, D, scale, False) else "dense"
 
 
 def attn_fwd_dense_flops(B, T, S, H, D):
@@ -221,7 +221,7 @@ def long_context_c3(steps: int = 5, warmup: int = 2, views: int = 64, topk: int 
     att_ms = statistics.mean(e[1].elapsed_time(e[2]) for e in evs)
     B, T, H, D = q.shape
     att_bytes = attn_fwd_algorithmic_bytes(B, T, H, D, topk)
-    attn_path = attn_fwd_path(T, topk, H, D)
+    attn_path = attn_fwd_path(B, T, topk, H, D)
 
     # The query-chunked stream (dsa_attention.py:1017-1283): same work, the indices and the
     # indexer workspace live per chunk of 16384 queries. Peak memory above the inputs.
@@ -628,7 +628,7 @@ def main() -> int:
     ap.add_argument("--no-sd", action="store_true", help="skip the approximate (source-downsample) top-k timing")
     ap.add_argument("--attn-path", choices=("auto", "dense", "gather"), default="auto",
                     help="attention forward without attn_sum: the masked dense pass, the gather kernel, "
-                         "or the automatic choice (dense below 15 K keys, union up to 96 K)")
+                         "or the automatic choice (dense below 15 K to 18 K keys, union up to 96 K)")
     ap.add_argument("--calibrate-copy", action="store_true",
                     help="also run 3 plain device copies of 1 GiB (reference kernel for rocprofv3 "
                          "FETCH_SIZE / WRITE_SIZE scaling)")
@@ -705,7 +705,7 @@ def main() -> int:
     att_avg = statistics.mean(att_ms)
     idx_avg = statistics.mean(idx_ms)
     att_gbs = att_bytes / (att_avg * 1e-3) / 1e9
-    attn_path = attn_fwd_path(T, Kk, H, D)
+    attn_path = attn_fwd_path(B, T, Kk, H, D)
     attn_flops = attn_fwd_dense_flops(B, T, Kk if attn_path == "union" else T, H, D)
     attn_tflops = attn_flops / (att_avg * 1e-3) / 1e12
     idx_tflops = idx_flops / (idx_avg * 1e-3) / 1e12

@@ -133,12 +133,17 @@ def _dense_fits(k: torch.Tensor, q_layout: str, seqlen_k: int, seqlen_q: int = 0
 
 
 # "auto" without attn_sum takes the union pass (gw_sparse_attn_fwd_union) in place of the dense
-# one where a query selects at most 1 / UNION_MIN_RATIO of the keys: sixteen queries then
-# select at most two thirds of them together. Measured in ms (16 heads, K = 1,024; dense, union):
-# S / K = 10.7 0.64, 0.73; 13.4 0.95, 1.02; 14.8 1.09, 1.10; 16.1 1.40, 1.36; 21.5 2.26, 1.83;
-# 32.2 4.7, 3.2; 42.9 7.4, 4.34; 85.9 28.2, 11.8.
+# one where a query selects at most 1 / UNION_MIN_RATIO of the keys: sixteen queries with
+# independent selections then select about two thirds of them together. Measured in ms (one
+# element, S queries, 16 heads, K = 1,024; dense, union): S / K = 10.7 0.64, 0.73; 13.4 0.95, 1.02;
+# 14.8 1.09, 1.10; 16.1 1.40, 1.36; 21.5 2.26, 1.83; 32.2 4.7, 3.2; 42.9 7.4, 4.34; 85.9 28.2,
+# 11.8. Where there are more rows or keys than UNION_FEW the chip is full with either, and the
+# line lies higher: 3 x 8,347 queries of 10,477 keys at S / K = 15.6 1.18, 1.26; 4 x 1,024 of 16,384
+# at 16.0 0.43, 0.45; 22,128 at 15.2 1.70, 1.78; 2 x 29,469 at 17.9 7.05, 6.76.
 # Beyond DENSE_MAX_RATIO the gather stays: it keeps P in fp32, both matrix-core passes in fp16.
 UNION_MIN_RATIO = 15
+UNION_MIN_RATIO_MANY = 18
+UNION_FEW = 16_500
 
 
 # "auto" with attn_sum runs the pass without it and then the mass from its lse
@@ -163,12 +168,15 @@ def _use_mass(batch: int, seqlen_q: int, seqlen_k: int, nheads: int, num_kv: int
     return seqlen_k <= ratio * num_kv and seqlen_k * num_kv >= MASS_MIN_WORK * nheads
 
 
-def _use_union(seqlen_k: int, num_kv: int, d: int, softmax_scale: float, return_attn: bool) -> bool:
+def _use_union(batch: int, seqlen_q: int, seqlen_k: int, num_kv: int, d: int, softmax_scale: float,
+               return_attn: bool) -> bool:
     if FORWARD_PATH not in ("auto", "union") or d != 64 or return_attn:
         return False
     if not 2.0 ** -58 <= softmax_scale <= 2.0 ** 58:
         return False
-    return FORWARD_PATH == "union" or UNION_MIN_RATIO * num_kv <= seqlen_k <= DENSE_MAX_RATIO * num_kv
+    few = batch * max(seqlen_q, seqlen_k) <= UNION_FEW
+    return (FORWARD_PATH == "union"
+            or (UNION_MIN_RATIO if few else UNION_MIN_RATIO_MANY) * num_kv <= seqlen_k <= DENSE_MAX_RATIO * num_kv)
 
 
 def _prep(x: torch.Tensor) -> torch.Tensor:
@@ -249,7 +257,8 @@ def _flash_attn_forward(
     # "auto" takes the union pass only in place of the dense one: a call beyond the dense limits
     # stays with the gather kernel.
     union = ((FORWARD_PATH == "union" or dense)
-             and _use_union(seqlen_k, num_kv, d, softmax_scale, attn_sum is not None and not separate_mass))
+             and _use_union(batch, seqlen_q, seqlen_k, num_kv, d, softmax_scale,
+                            attn_sum is not None and not separate_mass))
     if union:
         ws_bytes = int(lib.gw_sparse_attn_fwd_union_workspace_size(batch, seqlen_q, seqlen_k, nheads, d, num_kv))
         ws = torch.empty(max(ws_bytes, 1), device=q.device, dtype=torch.uint8)

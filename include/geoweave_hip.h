@@ -543,7 +543,8 @@ int gw_sparse_attn_fwd_dense_noalloc(int dtype,
  * attn_sum): the same results as gw_sparse_attn_fwd up to fp32 summation order and the fp16
  * rounding of P. Sixteen queries of a head form products with the keys that at least one of
  * them selected, 1 - (1 - K / S)^16 of all keys for spread selections; it pays off over
- * gw_sparse_attn_fwd_dense where a query selects less than about one key in eight.
+ * gw_sparse_attn_fwd_dense where a query selects less than about one key in fifteen (one in
+ * eighteen above 16,500 query rows or keys).
  * Needs D = 64 and softmax_scale * log2(e) in [2^-60, 2^60]; otherwise GW_ERR_UNSUPPORTED.
  * Queries that list a position twice, and batch elements with a non-finite K or V value, are
  * computed by the gather kernel inside this call. lse may be null.

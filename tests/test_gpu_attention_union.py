@@ -132,15 +132,20 @@ def test_layouts_strides_and_column_scales(gpu_device, layout):
         assert torch.equal(o2.float().cpu(), o) and torch.equal(lse2.cpu(), lse)
 
 
-def test_routes(gpu_device):
-    # The rule's own choice agrees with the gather kernel on both sides of its line.
-    for S, K in ((14 * 64, 64), (15 * 64, 64), (97 * 64, 64)):
-        print(f"[union] route S={S} K={K}", flush=True)
+def test_routes(gpu_device, monkeypatch):
+    # The rule's own choice gives the bits of the pass it names, and not those of the others.
+    cases = [(14, "dense", 16500), (15, "union", 16500), (97, "gather", 16500), (17, "dense", 14 * 64), (18, "union", 14 * 64)]
+    for ratio, path, few in cases:
+        S, K = ratio * 64, 64
+        monkeypatch.setattr(sifa, "UNION_FEW", few)
+        print(f"[union] route S={S} K={K} few={few}", flush=True)
         q, k, v = _inputs(1, 64, S, 2, torch.bfloat16, S)
         pos = _positions(1, 64, S, K, S)
         o, lse = _run(q, k, v, pos, path="auto")
-        og, lg = _run(q, k, v, pos, path="gather")
-        assert (o - og).norm() <= 2 * REL[torch.bfloat16] * og.norm() and (lse - lg).abs().max() < 1e-4
+        for name in ("dense", "union", "gather"):
+            on, ln = _run(q, k, v, pos, path=name)
+            assert torch.equal(o, on) == (name == path), (ratio, name)
+            assert (o - on).norm() <= 2 * REL[torch.bfloat16] * on.norm() and (lse - ln).abs().max() < 1e-4
 
 
 @pytest.mark.parametrize("limit,value", [("DENSE_MAX_S", 100), ("DENSE_MAX_T", 16), ("DENSE_MAX_K_ROW_STRIDE", 64)])

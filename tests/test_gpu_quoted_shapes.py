@@ -57,7 +57,8 @@ def test_metric_row_s32_indices_and_attention(gpu_device):
     # the bench's calls (bench.py: one step)
     idx, sc = sti.sparse_topk_indexer_inference_func(qi, ki, wi, qi.new_empty(0), 1024, 0.125, 256, 0,
                                                      return_scores=True)
-    assert sifa._use_dense(n, 1024, 16, 64, 0.125), "the metric row runs the masked dense pass"
+    assert sifa._use_dense(n, 1024, 16, 64, 0.125) and sifa._use_union(1, n, n, 1024, 64, 0.125, False), \
+        "the metric row runs the union pass"
     o, _, lse, _ = sifa._flash_attn_forward(q, k, v, idx, softmax_scale=0.125, return_attn=False)
     o_inf, _ = sifa.sparse_index_flash_attn_inference_func(q, k, v, idx, softmax_scale=0.125)
     torch.cuda.synchronize()
