@@ -21,6 +21,8 @@
 //   union_attn_kernel   - the attention.
 #include <math.h>
 
+#include <algorithm>
+#include <numeric>
 #include <type_traits>
 
 #include "gw_attn.h"
@@ -58,12 +60,12 @@ constexpr int kULMaxChunk = 136;  // tiles per chunk: 68 KB of query sets, two w
 
 __global__ __launch_bounds__(kULThreads) void union_lists_kernel(
     const int32_t* __restrict__ pos, int64_t psb, int64_t pst, int T, int S, int K, int ntiles, int chunk, int vec,
-    int vmax_words, int nqb, uint8_t* __restrict__ rec, int* __restrict__ flags,
+    int vmax_words, int nqb, int blk0, uint8_t* __restrict__ rec, int* __restrict__ flags,
     uint32_t* __restrict__ vmax, int* __restrict__ bad) {
   extern __shared__ __align__(16) uint32_t qset[];  // key s of the chunk: 16 bits of word s / 2
   __shared__ __align__(16) uint32_t slots[kULWaves][kUTile];  // per wave: row offset | query set << 16
   __shared__ int dup_any;
-  const int blk = blockIdx.x, b = blockIdx.y, nblk = gridDim.x;
+  const int blk = blk0 + blockIdx.x, b = blockIdx.y, nblk = gridDim.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int rows = min(kUQ, T - blk * kUQ);  // <= 0 for the padding blocks
   const int32_t* pblk = pos + b * psb + (int64_t)min(blk * kUQ, T - 1) * pst;
@@ -73,7 +75,7 @@ __global__ __launch_bounds__(kULThreads) void union_lists_kernel(
   }
   if (threadIdx.x == 0) dup_any = 0;
   bool dup = false;
-  uint8_t* brec = rec + ((int64_t)b * nblk + blk) * ntiles * kURec;
+  uint8_t* brec = rec + ((int64_t)b * nblk + blockIdx.x) * ntiles * kURec;
   for (int t0 = 0; t0 < ntiles; t0 += chunk) {
     const int nt = min(chunk, ntiles - t0);
     const int k0 = t0 * kUTile;
@@ -254,7 +256,8 @@ struct UnionParams {
   float* lse;
   int64_t qsb, qst, qsh;
   int64_t osb, ost, osh;
-  int T, H, nqb, ntiles, nblk;
+  int T, H, nqb, ntiles;
+  int blk0, nblk;  // the launch's 16-query blocks [blk0, blk0 + nblk), whose records rec holds
   float scale_log2;
 };
 
@@ -296,7 +299,7 @@ __global__ __launch_bounds__(1024) void union_attn_kernel(const UnionParams p) {
   const float sl2 = p.scale_log2;
   const int ntiles = p.ntiles;
 
-  int blk[NB];
+  int blk[NB];  // of the launch
   uint4 qb[NB][2];
   f32x4 acc[NB][4];
   float m[NB], l[NB];  // reference (exp2 domain; finite before the first selected key), row sum
@@ -304,8 +307,8 @@ __global__ __launch_bounds__(1024) void union_attn_kernel(const UnionParams p) {
 #pragma unroll
   for (int a = 0; a < NB; ++a) {
     blk[a] = (wg * nw + wave) * NB + a;
-    const int t = blk[a] * kUQ + i16;
-    const bool ok = t < p.T;
+    const int t = (p.blk0 + blk[a]) * kUQ + i16;
+    const bool ok = blk[a] < p.nblk && t < p.T;
     const uint16_t* qr = p.q + b * p.qsb + (int64_t)(ok ? t : 0) * p.qst + h * p.qsh + g * 8;
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
@@ -523,9 +526,9 @@ __global__ __launch_bounds__(1024) void union_attn_kernel(const UnionParams p) {
 #pragma unroll
   for (int a = 0; a < NB; ++a) {
     l[a] = pair_sum(row_sum(l[a]));
-    const int qb32 = blk[a] >> 1;
-    const int t = blk[a] * kUQ + i16;
-    bool active = t < p.T && p.bad[b] == 0;
+    const int qb32 = (p.blk0 + blk[a]) >> 1;
+    const int t = (p.blk0 + blk[a]) * kUQ + i16;
+    bool active = blk[a] < p.nblk && t < p.T && p.bad[b] == 0;
     if (qb32 < p.nqb) {
       const int* f = p.flags + ((int64_t)b * p.nqb + qb32) * 2;
       active &= (f[0] | f[1]) == 0;
@@ -554,19 +557,32 @@ __global__ __launch_bounds__(1024) void union_attn_kernel(const UnionParams p) {
 struct UnionLayout {
   size_t rec, flags, bad, vmax, tiles, total;
   int nqb, ntiles;
-  int64_t nblk;
+  int64_t nblk, chunk;  // 16-query blocks in all, and per launch
 };
+
+// The records of a launch hold at most this much; a call with more takes its queries in several
+// launches. They grow with T S: 1.94 GB at 87,936 queries and keys, where the dense pass's
+// selection words take half of that, 4.8 GB at 137,400, which is three launches.
+constexpr int64_t kURecBytes = 2ll << 30;
+constexpr int64_t kUCus = 256;
 
 UnionLayout union_layout(int64_t B, int64_t T, int64_t S, int64_t H) {
   UnionLayout L;
   const UnionListSizes u = union_list_sizes(T, S);
   L.ntiles = u.ntiles;
   L.nblk = u.nblk;
+  // A launch is whole workgroups of the largest shape (also whole 32-query blocks), and where the
+  // records of that many fit, as many as fill all CUs a whole number of times: each launch would
+  // else end with CUs idle (137,400 queries, K = 1,500: 29.0 ms in three equal launches, 27.3 so,
+  // 27.4 in one).
+  const int64_t unit = 2 * kUMaxWaves, round = unit * (kUCus / std::gcd(B * H, kUCus));
+  const int64_t fit = std::max<int64_t>(unit, kURecBytes / (B * L.ntiles * kURec) / unit * unit);
+  L.chunk = L.nblk <= fit ? L.nblk : fit < round ? fit : fit / round * round;
   L.nqb = (int)((T + 31) / 32);
   auto up = [](size_t x) { return (x + 255) / 256 * 256; };
   size_t o = 0;
   L.rec = o;
-  o = up(o + (size_t)B * L.nblk * L.ntiles * kURec);
+  o = up(o + (size_t)B * L.chunk * L.ntiles * kURec);
   L.flags = o;
   o = up(o + (size_t)B * L.nqb * 2 * 4);
   L.bad = o;
@@ -660,28 +676,12 @@ extern "C" int gw_sparse_attn_fwd_union(int dtype, const void* q, const int64_t*
   uint32_t* vmax = reinterpret_cast<uint32_t*>(ws + L.vmax);
   uint8_t* tiles = ws + L.tiles;
   const int in_fp16 = dtype == GW_DTYPE_FP16 ? 1 : 0;
-  {
-    const int vec = (K % 4 == 0 && pos_stride_t % 4 == 0 && pos_stride_b % 4 == 0 &&
-                     (reinterpret_cast<uintptr_t>(kv_pos) & 15) == 0)
-                        ? 1
-                        : 0;
-    const int nchunk = (L.ntiles + kULMaxChunk - 1) / kULMaxChunk;
-    const int chunk = (L.ntiles + nchunk - 1) / nchunk;
-    hipLaunchKernelGGL(union_lists_kernel, dim3((unsigned)L.nblk, (unsigned)B), dim3(kULThreads),
-                       (size_t)chunk * kUTile * 2, st, kv_pos, pos_stride_b, pos_stride_t, (int)T, (int)S, (int)K,
-                       L.ntiles, chunk, vec, (int)(H * 64), L.nqb, rec, flags, vmax, bad);
-    GW_HIP_LAUNCH_CHECK("union_lists_kernel launch");
-  }
-  hipLaunchKernelGGL(dense_vmax_kernel, dim3((unsigned)((S + kVmaxKeys - 1) / kVmaxKeys), (unsigned)H, (unsigned)B),
-                     dim3(256), 0, st, static_cast<const uint16_t*>(v), v_strides[0], v_strides[1], v_strides[2],
-                     static_cast<const uint16_t*>(k), k_strides[0], k_strides[1], k_strides[2], (int)S, (int)H,
-                     in_fp16, vmax, bad);
-  GW_HIP_LAUNCH_CHECK("dense_vmax_kernel launch");
-  hipLaunchKernelGGL(union_tiles_kernel, dim3((unsigned)(L.ntiles * 4), (unsigned)H, (unsigned)B), dim3(256), 0, st,
-                     static_cast<const uint16_t*>(k), k_strides[0], k_strides[1], k_strides[2],
-                     static_cast<const uint16_t*>(v), v_strides[0], v_strides[1], v_strides[2], (int)S, (int)H,
-                     L.ntiles, in_fp16, vmax, tiles);
-  GW_HIP_LAUNCH_CHECK("union_tiles_kernel launch");
+  const int vec = (K % 4 == 0 && pos_stride_t % 4 == 0 && pos_stride_b % 4 == 0 &&
+                   (reinterpret_cast<uintptr_t>(kv_pos) & 15) == 0)
+                      ? 1
+                      : 0;
+  const int passes = (L.ntiles + kULMaxChunk - 1) / kULMaxChunk;
+  const int tchunk = (L.ntiles + passes - 1) / passes;
   UnionParams p;
   p.q = static_cast<const uint16_t*>(q);
   p.tiles = tiles;
@@ -697,16 +697,38 @@ extern "C" int gw_sparse_attn_fwd_union(int dtype, const void* q, const int64_t*
   p.H = (int)H;
   p.nqb = L.nqb;
   p.ntiles = L.ntiles;
-  p.nblk = (int)L.nblk;
   p.scale_log2 = sl2;
-  const int64_t nblocks = (T + kUQ - 1) / kUQ;
-  const UnionShape u = union_shape(nblocks, H * B, 256);
-  const dim3 grid((unsigned)((nblocks + u.waves * u.nb - 1) / (u.waves * u.nb) * H), (unsigned)B);
-  if (dtype == GW_DTYPE_BF16)
-    launch_union_attn<BF16>(p, u, grid, st);
-  else
-    launch_union_attn<FP16>(p, u, grid, st);
-  GW_HIP_LAUNCH_CHECK("union_attn_kernel launch");
+  for (int64_t blk0 = 0; blk0 < L.nblk; blk0 += L.chunk) {
+    const int64_t nblk = std::min(L.chunk, L.nblk - blk0);
+    p.blk0 = (int)blk0;
+    p.nblk = (int)nblk;
+    hipLaunchKernelGGL(union_lists_kernel, dim3((unsigned)nblk, (unsigned)B), dim3(kULThreads),
+                       (size_t)tchunk * kUTile * 2, st, kv_pos, pos_stride_b, pos_stride_t, (int)T, (int)S, (int)K,
+                       L.ntiles, tchunk, vec, (int)(H * 64), L.nqb, p.blk0, rec, flags, vmax, bad);
+    GW_HIP_LAUNCH_CHECK("union_lists_kernel launch");
+    if (blk0 == 0) {
+      hipLaunchKernelGGL(dense_vmax_kernel, dim3((unsigned)((S + kVmaxKeys - 1) / kVmaxKeys), (unsigned)H, (unsigned)B),
+                         dim3(256), 0, st, static_cast<const uint16_t*>(v), v_strides[0], v_strides[1], v_strides[2],
+                         static_cast<const uint16_t*>(k), k_strides[0], k_strides[1], k_strides[2], (int)S, (int)H,
+                         in_fp16, vmax, bad);
+      GW_HIP_LAUNCH_CHECK("dense_vmax_kernel launch");
+      hipLaunchKernelGGL(union_tiles_kernel, dim3((unsigned)(L.ntiles * 4), (unsigned)H, (unsigned)B), dim3(256), 0, st,
+                         static_cast<const uint16_t*>(k), k_strides[0], k_strides[1], k_strides[2],
+                         static_cast<const uint16_t*>(v), v_strides[0], v_strides[1], v_strides[2], (int)S, (int)H,
+                         L.ntiles, in_fp16, vmax, tiles);
+      GW_HIP_LAUNCH_CHECK("union_tiles_kernel launch");
+    }
+    // Blocks with queries: at least one (the padding is less than one chunk's granule).
+    const int64_t nblocks = std::min(nblk, (T + kUQ - 1) / kUQ - blk0);
+    if (nblocks <= 0) break;
+    const UnionShape u = union_shape(nblocks, H * B, (int)kUCus);
+    const dim3 grid((unsigned)((nblocks + u.waves * u.nb - 1) / (u.waves * u.nb) * H), (unsigned)B);
+    if (dtype == GW_DTYPE_BF16)
+      launch_union_attn<BF16>(p, u, grid, st);
+    else
+      launch_union_attn<FP16>(p, u, grid, st);
+    GW_HIP_LAUNCH_CHECK("union_attn_kernel launch");
+  }
   return attn_fwd_flagged_blocks(dtype, q, q_strides, k, k_strides, v, v_strides, kv_pos, pos_stride_b, pos_stride_t,
                                  o, o_strides, lse, nullptr, B, T, S, H, D, K, softmax_scale, nullptr, 0, 0, 0, 0.f,
                                  nullptr, nullptr, 0, flags, bad, L.nqb, 2, stream);

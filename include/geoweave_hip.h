@@ -549,8 +549,9 @@ int gw_sparse_attn_fwd_dense_noalloc(int dtype,
  * Queries that list a position twice, and batch elements with a non-finite K or V value, are
  * computed by the gather kernel inside this call. lse may be null.
  * Workspace: gw_sparse_attn_fwd_union_workspace_size(B, T, S, H, D, K) bytes, 16-byte aligned
- * (selection records, B * round_up(T, 256) / 16 * ceil(S / 256) * 1024 bytes; the tiled K and
- * fp16 V, B * H * ceil(S / 256) * 65536 bytes; flags and |V| column maxima).
+ * (selection records, B * round_up(T, 256) / 16 * ceil(S / 256) * 1024 bytes, twice the dense
+ * pass's selection words, up to 2 GiB - beyond, the queries go in several launches; the tiled K
+ * and fp16 V, B * H * ceil(S / 256) * 65536 bytes; flags and |V| column maxima).
  * ------------------------------------------------------------------------------------ */
 size_t gw_sparse_attn_fwd_union_workspace_size(int64_t B, int64_t T, int64_t S, int64_t H, int64_t D,
                                                int64_t K);

@@ -218,3 +218,27 @@ def test_long_key_ranges(gpu_device, S):
     pos[0, 50, 3] = S - 1
     pos[0, 50, 4] = S - 1
     _against_gather(q, k, v, pos, list(range(0, T, 3)))
+
+
+def test_queries_in_several_launches(gpu_device):
+    # 100,000 queries and keys: records of 2.4 GiB, so two launches, of 65,536 and 34,464 queries.
+    T, K = 100_000, 1050
+    print(f"[union] {T} queries and keys", flush=True)
+    q, k, v = _inputs(1, T, T, 2, torch.bfloat16, 31)
+    g = torch.Generator().manual_seed(32)
+    off = torch.randint(0, T, (1, T, 1), generator=g).cuda()
+    pos = ((off + torch.arange(K, device="cuda") * 7919) % T).to(torch.int32)
+    pos[0, 65_530, 5] = pos[0, 65_530, 4]  # the gather kernel computes the blocks on both sides of the line
+    pos[0, 65_560, 5] = pos[0, 65_560, 4]
+    rows = list(range(65_500, 65_580, 5)) + [0, T - 1]
+    out = {}
+    for path in ("union", "gather"):
+        with _path(path):
+            o, _, lse, _ = sifa._flash_attn_forward(q.cuda(), k.cuda(), v.cuda(), pos, softmax_scale=0.125, return_attn=False)
+        out[path] = o.float(), lse
+    (o, lse), (og, lg) = out["union"], out["gather"]
+    rel = REL[torch.bfloat16] + 2.0 ** -9
+    assert (o - og).norm() <= rel * og.norm()
+    assert ((o - og).norm(dim=-1) <= 8 * rel * og.norm(dim=-1) + 1e-6).all()
+    assert (lse - lg).abs().max() <= 1e-4
+    _check(q[:, rows], k, v, pos[:, rows].cpu(), o[:, rows].cpu(), lse[:, rows].cpu())
