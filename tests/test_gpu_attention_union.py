@@ -242,3 +242,33 @@ def test_queries_in_several_launches(gpu_device):
     assert ((o - og).norm(dim=-1) <= 8 * rel * og.norm(dim=-1) + 1e-6).all()
     assert (lse - lg).abs().max() <= 1e-4
     _check(q[:, rows], k, v, pos[:, rows].cpu(), o[:, rows].cpu(), lse[:, rows].cpu())
+
+
+def test_captured_in_a_graph(gpu_device):
+    # The union pass, and the forward with the separate mass, captured and replayed between eager work.
+    print("[union] graph", flush=True)
+    for S, K, attn in ((1100, 60, False), (1300, 260, True)):
+        q, k, v = (x.cuda() for x in _inputs(1, 300, S, 4, torch.bfloat16, S))
+        pos = _positions(1, 300, S, K, S).cuda()
+        assert sifa._use_mass(1, 300, S, 4, K) if attn else sifa._use_union(1, 300, S, K, 64, 0.125, False)
+
+        def call():
+            return sifa._flash_attn_forward(q, k, v, pos, softmax_scale=0.125, return_attn=attn)[:3]
+
+        eager = call()
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            call()
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            captured = call()
+        for i in range(4):
+            for t in captured:
+                if t is not None:
+                    t.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert all(a is b is None or torch.equal(a, b) for a, b in zip(eager, captured)), (S, i)
+            assert torch.equal(call()[0], eager[0])

@@ -64,12 +64,28 @@ def test_row_forms(gpu_device, dtype, H, T):
 
 
 def test_rows_with_too_few_finite_scores_and_nan(gpu_device):
-    # Fewer unmasked keys than top-k, and NaN scores: the rows go to the exact fallback on both
-    # paths.
+    # The even rows have 50 unmasked keys for a top-k of 100: both paths send them to the exact
+    # fallback. The odd rows are selected from, NaN scores among them (from gates and from the mask,
+    # of both signs): a positive NaN ranks above every number, a negative one is not a candidate. Their
+    # selection is the fallback's, to which the forced threshold of +inf sends every row.
     print("[rows] masked, NaN", flush=True)
     q, k, w = _inputs(1, 40, 700, 4, torch.bfloat16, 9)
     mask = torch.zeros(1, 40, 700)
     mask[:, ::2, 50:] = float("-inf")
+    mask = mask.bfloat16().cuda()
+    nan, minus = torch.tensor([0x7FC0, -0x40], dtype=torch.int16).view(torch.bfloat16).cuda()
+    w[0, 300], w[0, 301] = nan, minus
+    mask[:, :, 400], mask[:, :, 401] = nan, minus
     k[0, 5, 0, 0] = float("nan")
-    a, b = _both(q, k, w, mask.cuda(), 100)
-    assert torch.equal(a[0].sort(-1).values, b[0].sort(-1).values)
+    a, b = _both(q, k, w, mask, 100)
+    exact = sti.indexer_topk_forward(q, k, w, mask, 100, 0.125, flags=sti.FLAG_TAU_PLUS_INF)
+    torch.cuda.synchronize()
+    order = [x[0].sort(-1).values for x in (a, b, exact)]
+    assert torch.equal(order[0], order[1]) and torch.equal(order[0][:, 1::2], order[2][:, 1::2])
+    odd = order[0][:, 1::2]
+    assert ((odd == 300).any(-1) & (odd == 400).any(-1)).all()
+    assert not ((odd == 301) | (odd == 401)).any()
+    # the scores, the two NaN entries aside, are the fallback's too (its fp32 dot products round
+    # in another order: one bf16 rounding apart at most)
+    top = [x[1].float()[:, 1::2].nan_to_num(nan=0.0).sort(-1).values for x in (a, exact)]
+    assert ((top[0] - top[1]).abs() <= 2.0 ** -7 * top[1].abs()).all()
