@@ -749,8 +749,8 @@ def main() -> int:
         "attn_fwd_ms": round(att_avg, 3),
         "attn_path": attn_path,
         # The roofline of what runs: the masked dense pass against the matrix cores on
-        # the flops it executes, the union pass on the selected products alone (it is bound by
-        # the instructions around them), the gather kernel against HBM on the bytes it gathers.
+        # the flops it executes, the union pass on the selected products alone ("limited_by" names
+        # what holds it below), the gather kernel against HBM on the bytes it gathers.
         "roofline": ({
             "kernel": ("union_attn_kernel (one attention call: + union_lists_kernel, union_tiles_kernel, "
                        "dense_vmax_kernel)" if attn_path == "union" else
@@ -763,6 +763,8 @@ def main() -> int:
             "frac": round(attn_tflops / MFMA_BF16_PEAK_TFLOPS, 4),
             "traffic": traffic,
             "algorithmic_flops": attn_flops,
+            **({"limited_by": "VALU issue: the instructions around the products of a block's key union"}
+               if attn_path == "union" else {}),
         } if attn_path != "gather" else {
             "kernel": "sparse_attn_fwd_kernel",
             "bound": "hbm",

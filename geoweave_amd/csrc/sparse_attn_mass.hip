@@ -9,17 +9,17 @@
 // without, and 167 us for the sum). Here a second pass recomputes: a wave owns 32 queries x 128
 // keys, keeps their sums over the heads in registers, and per head forms S^T = K Q^T on the
 // matrix cores and adds exp2(s * scale log2 e - lse2) - no selection, no V, no row sums. The
-// sums go to a score matrix of a chunk of queries, small enough to stay in the last-level cache,
+// sums go to a score matrix of a chunk of queries, at most 256 MiB or one workgroup's queries,
 // from which attn_mass_gather_kernel takes the selected ones. A value that is not selected is
 // never read, so it needs no mask (also where it overflows or a key row is not finite).
 //
-// Sixteen waves share the head's K tile in LDS, four a SIMD at 120 registers. Bound (10,992
-// keys, 0.80 ms with the gather): latency; the VALU, which a pair and head costs an FMA, an
-// exponential and an add, is active 49 % of the time, the matrix cores 21 %, and a timing copy
-// without the copies to LDS, or without the exponentials, is 10-14 % faster. Eight waves of two
+// Sixteen waves share the head's K tile in LDS, four a SIMD at 120 registers. Bound: latency; the
+// VALU, which a pair and head costs an FMA, an exponential and an add, is active 46 % of the
+// cycles, the matrix cores 20 % (counters at 9,384 keys), and a timing copy without the copies to
+// LDS, or without the exponentials, is 10-14 % faster. Eight waves of two
 // 32-query blocks (232 registers) took 6.9 against 6.3 ms at 32,976 keys, their query operands
-// read by the lanes instead of staged 7.6. At 5,496 keys this kernel takes 147 us and the gather 37;
-// the whole forward with the mass 0.67 -> 0.40 ms, at 10,992 keys 1.52 -> 1.23 ms.
+// read by the lanes instead of staged 7.6. At 5,496 keys this kernel takes 141 us and the gather 28;
+// the whole forward with the mass 0.56 -> 0.37 ms against the stored scores, at 10,992 keys 1.31 -> 1.23.
 #include <math.h>
 
 #include "gw_common.h"
@@ -31,7 +31,7 @@ namespace {
 constexpr int kMWaves = 16;
 constexpr int kMKeys = 128;                // keys per tile
 constexpr int kMRows = kMWaves * 32;       // queries per workgroup
-constexpr int64_t kMChunkBytes = 256ll << 20;  // score matrix of one chunk of queries
+constexpr int64_t kMChunkBytes = 256ll << 20;  // score matrix of one chunk of query groups
 constexpr int kMassMaxK = 1024;            // a row's values sit in registers in the gather
 
 struct MassParams {

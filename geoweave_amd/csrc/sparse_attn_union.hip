@@ -6,8 +6,9 @@
 // keys selected per query that is 1 - (1 - r)^16 of them (31 % at 1,024 of 43,968 keys, 17 %
 // at 1,024 of 87,936), so matrix work, exponentials and operand reads all shrink by that
 // factor, while each K and V row is still read from memory once per workgroup (up to 512
-// queries) and shared through LDS. With 16 heads the whole call takes 4.34 ms against the
-// dense pass's 7.45 ms at 43,968 keys (K = 1,024) and 11.8 ms against 28.4 ms at 87,936.
+// queries) and shared through LDS. With 16 heads and selections drawn independently the whole call
+// takes 4.34 ms against the dense pass's 7.45 at 43,968 keys (K = 1,024) and 11.8 against 28.4 at
+// 87,936; with an indexer's selections, which share more keys, 3.93 and 11.6.
 //
 // Pieces (all on the caller's stream):
 //   union_lists_kernel  - the (block, tile) records of gw_union.h from the positions; a position
@@ -222,14 +223,15 @@ __global__ __launch_bounds__(256) void union_tiles_kernel(const uint16_t* __rest
 // The reference maximum is lazy, as in the masked dense pass: it moves only when a lane's
 // weights of a step sum to more than kUSumCap.
 //
-// Bound (43,968 keys, 16 waves of one block each): VALU issue. A step of a wave takes 304
-// cycles of its SIMD, about 60 VALU and 8 matrix instructions (matrix cores 128 cycles, LDS
-// 60 of the CU's); a tile costs a further 1,400 cycles in which the 16 waves leave the barrier,
-// queue for their first operands and drain. Sixteen queries a block rather than 32: the union
-// of 32 queries is 1.7 times as large at these sizes, so the exponentials grow by that while
-// only the LDS reads shrink. Tiles of 256 keys: the largest that fit twice. Lists through
-// buffer loads two tiles ahead (a flat load also counts as an LDS access, and every operand
-// read waits for it). A tile's last step takes 16 slots when the rest are empty (4.6 -> 4.34 ms).
+// Bound (43,968 keys, 16 waves of one block each): VALU issue. A wave issues about 65 VALU and 8
+// matrix instructions a step; by the counters a SIMD issues VALU 65 % of the cycles and its
+// matrix core is busy 29 %, 38 % of that beside VALU. Part of the rest is the end of a tile, where
+// the waves, of different step counts, meet at the barrier and queue for their first operands.
+// Sixteen queries a block rather than 32: the union of 32 queries is 1.7 times as large at these
+// sizes, so the exponentials grow by that while only the LDS reads shrink. Tiles of 256 keys: the
+// largest that fit twice. Lists through buffer loads two tiles ahead (a flat load also counts as
+// an LDS access, and every operand read waits for it). A tile's last step takes 16 slots when the
+// rest are empty (4.6 -> 4.34 ms).
 // Measured and not kept: the selection as a 4-bit-float matrix product instead of eight bit
 // selects a step (4.52 ms: the product sits at the head of the step's dependent chain).
 // ---------------------------------------------------------------------------------------

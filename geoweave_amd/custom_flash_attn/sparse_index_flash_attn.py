@@ -108,7 +108,7 @@ def _pad_head_dim(x: torch.Tensor, dp: int) -> torch.Tensor:
 
 # Forward: "auto" picks the masked dense pass (gw_sparse_attn_fwd_dense) when a query
 # selects at least 1 / DENSE_MAX_RATIO of the keys (and, with attn_sum, K <=
-# DENSE_ATTN_SUM_MAX_K), "dense" / "gather" force one path (tests and measurements). The
+# DENSE_ATTN_SUM_MAX_K), "dense" / "gather" / "union" force one path (tests and measurements). The
 # dense pass costs ~ T·S, the gather ~ T·K: on MI355X they break even near S = 124·K.
 # The dense kernel's 32-bit load offsets bound the K token stride and S, its grid of at most
 # 65535 query blocks (whole workgroups of 8) bounds T (DENSE_MAX_*).
